@@ -6,6 +6,7 @@
 #include <cstring>
 #include <memory>
 #include <numeric>
+#include <type_traits>
 
 #include "cpml2d.h"
 #include "devbuf.h"
@@ -20,112 +21,234 @@ namespace sssi {
 // (fwdTimeSpongeFor2dAw.m:83-92); the stored level carries one factor and the
 // second is applied when it is read back as p_old.
 struct Sponge2dArgs {
-    const float *pcur;
-    float *pold;
+    const float *pcur, *pold;  // levels before the first step
+    float *ocur, *oold;        // levels after the last one (other buffers)
     const float *vdt;
     const float *g;  // g[m], m < nB
     int nz, nx, pitch, rows, nB;
     float idx2, idz2;  // 1/dx^2, 1/dz^2
+    // time index of the first step and its direction, number of steps (<= kSpK)
+    int t0, reverse, nsteps;
     const int *src_cell;
-    const float *src_amp;
-    int nsrc;
-    const float *surf;
-    float *rec;
-    float *snap;
+    const float *src_amp;  // [t*nsrc + k], t < src_nt (forward)
+    int nsrc, src_nt;
+    const float *surf;  // [t*nx + j], t < surf_nt (reverse)
+    int surf_nt;
+    float *rec;   // [t*nx + j] or null
+    float *snap;  // slices at t % snap_stride == 0, slot t/stride - slot0; or null
+    int snap_stride;
+    int64_t snap_slot0;
     int *health;  // non-finite watchdog word (top row), or null
-    int step;     // launch step reported to it
+    int step;     // launch step reported to it (of the first step)
 };
 
-// Rows per wavefront of the sponge step; a block is 4 wavefronts stacked in z.
-// At 1040 x 3080 with the XCD-banded tile order below, us per step at 1, 2, 4,
-// 8, 16 rows: 13.9, 9.2, 7.4, 7.9, 9.4.
-constexpr int kSpRZ = 4;
+// Steps per launch of the sponge kernel, and the rows of its tile (64 columns
+// wide); the inner cells are what a tile writes.
+constexpr int kSpK = 8, kSpZ = 32;
+constexpr int kSpCX = kTX - 2 * kSpK, kSpCZ = kSpZ - 2 * kSpK;
 
-// A wavefront owns 64 columns x kSpRZ rows (lane = column).  Every load is a
-// raw buffer load with the wave-uniform row offset in the scalar offset: the
-// column window p(i0-1 .. i0+kSpRZ) once, the x neighbours as loads shifted by
-// one column, then p_old and v*dt.  Rows i0-1 .. i0+kSpRZ and columns j-1 ..
-// j+1 of every wavefront that has a row inside the model lie in the padded
-// array (16 rows above, at least 32 below the interior rounded up to 64 rows,
-// 32 columns each side).  Lanes outside the model store nothing, so the zero
-// padding read as the boundary stays zero.
-// The launch is 1-D over ntx * ntz block tiles (x fastest).  Block b runs on
-// XCD b % 8, so block b takes tile t of XCD b % 8's contiguous band of the
-// tile list: row neighbours then share one L2 for the rows between them.
-template <int RZ>
-__global__ void __launch_bounds__(256) sponge2d_step(Sponge2dArgs a, int ntx) {
+// Value of the lane before / after (DPP wave_shr:1 / wave_shl:1), 0 at the
+// wavefront's edge.
+__device__ __forceinline__ float lane_left(float v) {
+    return __int_as_float(
+        __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_right(float v) {
+    return __int_as_float(
+        __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130, 0xf, 0xf, true));
+}
+
+// Up to kSpK steps on the tile (ty, tx): see sponge2d_steps.  INNER: the whole
+// tile lies inside the model and off its top row, and no damping strip touches
+// it (every factor 1).
+template <int R, bool INNER>
+__device__ __forceinline__ void sponge2d_tile(const Sponge2dArgs &a, int tx, int ty,
+                                              float (&edge)[2][kSpZ / R + 2][2][64]) {
+    constexpr int K = kSpK;
     const int lane = threadIdx.x & 63, w = wave_id();
+    const int j = tx * kSpCX - K + lane;
+    const int q0 = w * R;                   // the wave's first row in the tile
+    const int i0 = ty * kSpCZ - K + q0;     // and in the model
+    const bool jin = INNER || (j >= 0 && j < a.nx);
+    const bool jmine = jin && lane >= K && lane < 64 - K;
+    const uint32_t rowb = (uint32_t)a.pitch * 4u;
+    const uint32_t nbytes = rowb * (uint32_t)a.rows;
+    const uint32_t vcol = jin ? (uint32_t)(j + kHX) * 4u : kOOB;
+    auto iin = [&](int r) { return INNER || (i0 + r >= 0 && i0 + r < a.nz); };
+    auto mine = [&](int r) { return iin(r) && q0 + r >= K && q0 + r < kSpZ - K; };
+    auto srow = [&](int r) { return (uint32_t)(i0 + r + kHZ) * rowb; };
+
+    float pa[R], pb[R], ax[R], az[R], gf[R];  // p (even steps), p_old, factors
+    {
+        const __amdgpu_buffer_rsrc_t rP = buf_rsrc(a.pcur, nbytes);
+        const __amdgpu_buffer_rsrc_t rO = buf_rsrc(a.pold, nbytes);
+        const __amdgpu_buffer_rsrc_t rV = buf_rsrc(a.vdt, nbytes);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            // rows outside the model: every lane out of range, so 0
+            const uint32_t v = iin(r) ? vcol : kOOB, so = iin(r) ? srow(r) : 0u;
+            pa[r] = buf_ld(rP, v, so);
+            pb[r] = buf_ld(rO, v, so);
+            ax[r] = buf_ld(rV, v, so);
+        }
+    }
+    // all ones in the lanes and rows inside the model: ANDed to the update, it
+    // keeps the cells outside 0 without a branch
+    int keep[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) keep[r] = jin && iin(r) ? -1 : 0;
+    // damping factor: the bottom strip's by row, else the side strips' by column
+    float gx = 1.f;
+    if constexpr (!INNER) {
+        if (jin && j < a.nB) gx = a.g[j];
+        else if (jin && j >= a.nx - a.nB) gx = a.g[a.nx - 1 - j];
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float v2 = ax[r] * ax[r];
+        ax[r] = v2 * a.idx2;
+        az[r] = v2 * a.idz2;
+        gf[r] = gx;
+        if constexpr (!INNER)
+            if (iin(r) && i0 + r >= a.nz - a.nB) gf[r] = ld_uniform(a.g + (a.nz - 1 - i0 - r));
+    }
+    // sources in this wave's rows and columns
+    bool has_src = false;
+    if (!a.reverse)
+        for (int k = 0; k < a.nsrc; ++k) {
+            const int cell = ld_uniform(a.src_cell + k);
+            const int ci = cell / a.nx, cj = cell - ci * a.nx;
+            has_src |= ci >= i0 && ci < i0 + R && cj >= tx * kSpCX - K && cj < tx * kSpCX - K + 64;
+        }
+    const bool top = !INNER && i0 <= 0 && i0 + R > 0;  // the wave holds row 0
+    const bool surf_here = top && a.reverse && a.surf;
+
+    // source terms of a step, summed per cell in source order, then surface injection
+    auto sources = [&](int t, float (&sv)[R]) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) sv[r] = 0.f;
+        if (has_src && t < a.src_nt)
+            for (int k = 0; k < a.nsrc; ++k) {
+                const int cell = ld_uniform(a.src_cell + k);
+                const int ci = cell / a.nx, cj = cell - ci * a.nx;
+                const float amp = ld_uniform(a.src_amp + (size_t)t * a.nsrc + k);
+                if (cj == j) {
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (ci == i0 + r) sv[r] += amp;
+                }
+            }
+        if (surf_here && t < a.surf_nt) {
+            const float x = jin ? a.surf[(size_t)t * a.nx + j] : 0.f;
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (i0 + r == 0) sv[r] += x;
+        }
+    };
+    const bool driven = has_src || surf_here;  // wave-uniform
+    auto update = [&](float (&p)[R], float (&q)[R], float up, float below, int t, auto src) {
+        float sv[R];
+        if constexpr (src) sources(t, sv);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float pc = p[r], dn = r + 1 < R ? p[r + 1] : below;
+            // b p - p_old + ax (pR+pL) + az (pD+pU) regrouped as
+            // p + (p - p_old) + ax((pR-p)+(pL-p)) + az((pD-p)+(pU-p)): the FP32
+            // rounding then scales with the increments instead of with 2p.
+            float lap = fmaf(ax[r], (lane_right(pc) - pc) + (lane_left(pc) - pc),
+                             az[r] * ((dn - pc) + (up - pc)));
+            if constexpr (src) {
+                const float vd = iin(r) && jin ? a.vdt[(size_t)(i0 + r + kHZ) * a.pitch + j + kHX]
+                                               : 0.f;
+                lap = fmaf(-sv[r], vd * vd, lap);
+            }
+            float pn = pc + (lap + (INNER ? pc - q[r] : fmaf(-gf[r], q[r], pc)));
+            if constexpr (!INNER) {
+                pn *= gf[r];
+                pn = __int_as_float(__float_as_int(pn) & keep[r]);
+            }
+            q[r] = pn;
+            up = pc;
+        }
+    };
+    auto step = [&](int s, float (&p)[R], float (&q)[R]) {
+        const int t = a.reverse ? a.t0 - s : a.t0 + s;
+        float (&E)[kSpZ / R + 2][2][64] = edge[s & 1];
+        E[w + 1][0][lane] = p[0];
+        E[w + 1][1][lane] = p[R - 1];
+        __syncthreads();
+        const float up = E[w][1][lane], below = E[w + 2][0][lane];
+        if (driven) update(p, q, up, below, t, std::true_type{});
+        else update(p, q, up, below, t, std::false_type{});
+        if (top) {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (i0 + r == 0 && mine(r)) {
+                    if (a.rec && jmine) a.rec[(size_t)t * a.nx + j] = q[r];
+                    if (a.health) report_nonfinite(a.health, jmine && nonfinite(q[r]), a.step + s);
+                }
+        }
+        if (a.snap && t % a.snap_stride == 0) {
+            const __amdgpu_buffer_rsrc_t rS = buf_rsrc(
+                a.snap + (size_t)(t / a.snap_stride - a.snap_slot0) * a.nz * a.nx,
+                (uint32_t)a.nz * (uint32_t)a.nx * 4u);
+            const uint32_t vs = jmine ? (uint32_t)j * 4u : kOOB;
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                buf_st(q[r], rS, mine(r) ? vs : kOOB,
+                       mine(r) ? (uint32_t)(i0 + r) * (uint32_t)a.nx * 4u : 0u);
+        }
+    };
+#pragma unroll 1
+    for (int s = 0; s + 1 < a.nsteps; s += 2) {
+        step(s, pa, pb);
+        step(s + 1, pb, pa);
+    }
+    const bool odd = a.nsteps & 1;
+    if (odd) step(a.nsteps - 1, pa, pb);  // the newest level ends in pb
+    const __amdgpu_buffer_rsrc_t wP = buf_rsrc(odd ? a.oold : a.ocur, nbytes);
+    const __amdgpu_buffer_rsrc_t wO = buf_rsrc(odd ? a.ocur : a.oold, nbytes);
+    const uint32_t vst = jmine ? vcol : kOOB;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t v = mine(r) ? vst : kOOB, so = mine(r) ? srow(r) : 0u;
+        buf_st(pa[r], wP, v, so);
+        buf_st(pb[r], wO, v, so);
+    }
+}
+
+// nsteps <= kSpK time steps per launch.  A workgroup holds a tile of kSpZ rows
+// x 64 columns in registers (lane = column, R rows per wavefront) and steps it
+// without going back to memory: x neighbours by DPP, z neighbours from the
+// lane's own registers and, at a wavefront's first and last row, through LDS
+// (double-buffered, one barrier per step).  Cells at the tile's edge miss a
+// neighbour and go wrong, and each step moves that error one cell inwards, so
+// the tile's inner kSpCZ x kSpCX cells are exact after nsteps <= kSpK steps
+// and are what it writes: two levels into buffers other than those it reads,
+// as its neighbours still read their halos there.  Cells outside the model
+// stay 0, which is the boundary.
+// One step per launch was bound by the launch on small grids and by streaming
+// four arrays per step on large ones; here 8 steps share a launch and one
+// trip, at 12 VALU instructions per cell and step and 2.7 times the cells.
+// 800 steps, whole call, one step per launch / this kernel: 100 x 150 2.59 /
+// 1.14 ms, 301 x 450 with 58 snapshots 3.8 / 2.8, 515 x 1203 5.0 / 2.85,
+// 1040 x 3080 12.0 / 8.3 (4 of them the model's way to the device).
+// R = 4 (8 waves) has the shorter step, R = 8 (4 waves) the better use of a
+// full chip: 100 x 150 1.14 against 1.50 ms, 515 x 1203 3.43 against 2.85.
+// Blocks are 1-D over the tiles, XCD-banded: block b runs on XCD b % 8 and
+// takes the next tile of that XCD's contiguous band.
+template <int R>
+__global__ void __launch_bounds__(64 * kSpZ / R) sponge2d_steps(Sponge2dArgs a, int ntx) {
+    __shared__ float edge[2][kSpZ / R + 2][2][64];
     const int nb = (int)gridDim.x, b = (int)blockIdx.x;
     const int q = nb / 8, rem = nb % 8, x = b % 8;
     const int t = x * q + min(x, rem) + b / 8;
     const int ty = t / ntx, tx = t - ty * ntx;
-    const int j = tx * 64 + lane;
-    const int i0 = (ty * 4 + w) * RZ;
-    if (i0 >= a.nz) return;
-    const bool jin = j < a.nx;
-    const uint32_t rowb = (uint32_t)a.pitch * 4u;
-    const uint32_t nbytes = rowb * (uint32_t)a.rows;
-    const __amdgpu_buffer_rsrc_t rP = buf_rsrc(a.pcur, nbytes);
-    const __amdgpu_buffer_rsrc_t rO = buf_rsrc(a.pold, nbytes);
-    const __amdgpu_buffer_rsrc_t rV = buf_rsrc(a.vdt, nbytes);
-    const uint32_t vcol = (uint32_t)(j + kHX) * 4u;
-    const uint32_t srow = (uint32_t)(i0 + kHZ) * rowb;
-
-    float col[RZ + 2], cl[RZ], cr[RZ], po[RZ], vd[RZ];
-#pragma unroll
-    for (int r = 0; r < RZ + 2; ++r) col[r] = buf_ld(rP, vcol, srow + (r - 1) * rowb);
-#pragma unroll
-    for (int r = 0; r < RZ; ++r) {
-        cl[r] = buf_ld(rP, vcol - 4u, srow + r * rowb);
-        cr[r] = buf_ld(rP, vcol + 4u, srow + r * rowb);
-        po[r] = buf_ld(rO, vcol, srow + r * rowb);
-        vd[r] = buf_ld(rV, vcol, srow + r * rowb);
-    }
-
-    // damping factor: the bottom strip's by row, else the side strips' by column
-    const int nB = a.nB;
-    float gx = 1.f;
-    if (jin && j < nB) gx = a.g[j];
-    else if (jin && j >= a.nx - nB) gx = a.g[a.nx - 1 - j];
-    // source terms, summed per cell in source order, then surface injection
-    float s[RZ];
-#pragma unroll
-    for (int r = 0; r < RZ; ++r) s[r] = 0.f;
-    for (int k = 0; k < a.nsrc; ++k) {
-        const int cell = ld_uniform(a.src_cell + k);
-        const int ci = cell / a.nx, cj = cell - ci * a.nx;
-        if (ci >= i0 && ci < i0 + RZ && cj == j) {
-            const float amp = ld_uniform(a.src_amp + k);
-#pragma unroll
-            for (int r = 0; r < RZ; ++r)
-                if (ci == i0 + r) s[r] += amp;
-        }
-    }
-    if (a.surf && i0 == 0 && jin) s[0] += a.surf[j];
-
-    float pn0 = 0.f;
-#pragma unroll
-    for (int r = 0; r < RZ; ++r) {
-        const int i = i0 + r;
-        if (i >= a.nz) break;
-        const float gf = i >= a.nz - nB ? ld_uniform(a.g + (a.nz - 1 - i)) : gx;
-        const float v2 = vd[r] * vd[r];
-        const float ax = v2 * a.idx2, az = v2 * a.idz2;
-        // b p - p_old + ax (pR+pL) + az (pD+pU) regrouped as
-        // p + (p - p_old) + ax((pR-p)+(pL-p)) + az((pD-p)+(pU-p)): the FP32
-        // rounding then scales with the increments instead of with 2p.
-        const float pc = col[r + 1];
-        const float lap = ax * ((cr[r] - pc) + (cl[r] - pc)) + az * ((col[r + 2] - pc) + (col[r] - pc));
-        float pn = pc + ((pc - gf * po[r]) + (lap - v2 * s[r]));
-        pn *= gf;
-        buf_st(pn, rO, jin ? vcol : kOOB, srow + r * rowb);
-        if (r == 0) pn0 = pn;
-        if (jin) {
-            if (a.rec && i == 0) a.rec[j] = pn;
-            if (a.snap) a.snap[(size_t)i * a.nx + j] = pn;
-        }
-    }
-    if (a.health && i0 == 0) report_nonfinite(a.health, jin && nonfinite(pn0), a.step);
+    const int z0 = ty * kSpCZ - kSpK, x0 = tx * kSpCX - kSpK;  // first row and column held
+    if (z0 > 0 && z0 + kSpZ <= a.nz - a.nB && x0 >= a.nB && x0 + 64 <= a.nx - a.nB)
+        sponge2d_tile<R, true>(a, tx, ty, edge);
+    else
+        sponge2d_tile<R, false>(a, tx, ty, edge);
 }
 
 // ---------------------------------------------------------------------------
@@ -140,10 +263,10 @@ class Prop2D final : public Prop {
     int64_t done = 0;  // steps since reset (parity of the current level)
     // sponge
     int64_t pitch = 0, rows = 0;
-    DevBuf<float> sp[2], vdt, gtab;
+    // levels in pairs (current, old): a launch reads one pair, writes the other
+    DevBuf<float> sp[2][2], vdt, gtab;
     DevBuf<int> sp_health;
-    std::vector<int> h_cells;
-    int cur = 0;
+    int cur = 0;  // pair that holds the present levels
 
     Prop2D(const double *v, int64_t nz_, int64_t nx_, int abc_, int N_, int nB_, double dz_,
            double dx_, double dt_) {
@@ -166,8 +289,8 @@ class Prop2D final : public Prop {
             pitch = round_up(kHX + round_up(nx, kTX) + 32, 64);
             rows = kHZ + round_up(nz, kTZmax) + kHZbot;
             const size_t np = (size_t)pitch * rows;
-            sp[0].alloc(np);
-            sp[1].alloc(np);
+            for (auto &pair : sp)
+                for (auto &level : pair) level.alloc(np);
             vdt.alloc(np);
             upload_model(v, nz, nx, 1, dt, false, vdt.p, vdt.n, pitch, 0, kHZ, 0, kHX, stream);
             std::vector<float> gg(std::max(nB, 1), 1.f);
@@ -269,8 +392,9 @@ class Prop2D final : public Prop {
         if (g) {
             g->zero_state(stream);
         } else {
-            SSSI_HIP(hipMemsetAsync(sp[0].p, 0, sp[0].bytes(), stream));
-            SSSI_HIP(hipMemsetAsync(sp[1].p, 0, sp[1].bytes(), stream));
+            for (auto &pair : sp)
+                for (auto &level : pair)
+                    SSSI_HIP(hipMemsetAsync(level.p, 0, level.bytes(), stream));
             arm_health(sp_health.p, stream);
         }
         done = 0;
@@ -365,32 +489,52 @@ class Prop2D final : public Prop {
 
     void scan_field() override {
         if (g) g->scan_nonfinite((int)(done & 1), (int)done, stream);
-        else launch_nonfinite_scan(sp[cur].p, sp[cur].n, sp_health.p, (int)done, stream);
+        else launch_nonfinite_scan(sp[cur][0].p, sp[cur][0].n, sp_health.p, (int)done, stream);
     }
 
-    void step_sponge(int64_t t, bool reverse, bool record, float *snap, int step) {
+    // n <= kSpK sponge steps from time index t
+    void steps_sponge(int64_t t, int n, bool reverse, bool record, const SnapSink *sink,
+                      int step) {
         Sponge2dArgs a{};
         a.health = sp_health.p;
         a.step = step;
-        a.pcur = sp[cur].p;
-        a.pold = sp[cur ^ 1].p;
+        a.pcur = sp[cur][0].p;
+        a.pold = sp[cur][1].p;
+        a.ocur = sp[cur ^ 1][0].p;
+        a.oold = sp[cur ^ 1][1].p;
         a.vdt = vdt.p;
         a.g = gtab.p;
         a.nz = (int)nz; a.nx = (int)nx; a.pitch = (int)pitch; a.rows = (int)rows; a.nB = nB;
         a.idx2 = (float)(1.0 / (dx * dx));
         a.idz2 = (float)(1.0 / (dz * dz));
-        if (!reverse && nsrc > 0 && t < src_nt) {
+        a.t0 = (int)t;
+        a.reverse = reverse ? 1 : 0;
+        a.nsteps = n;
+        if (!reverse && nsrc > 0) {
             a.src_cell = src_cell.p;
-            a.src_amp = src_amp.p + (size_t)t * nsrc;
+            a.src_amp = src_amp.p;
             a.nsrc = nsrc;
+            a.src_nt = (int)src_nt;
         }
-        if (reverse && surf.p && t < surf_nt) a.surf = surf.p + (size_t)t * nx;
-        if (record) a.rec = rec.p + (size_t)t * nx;
-        a.snap = snap;
-        const int ntx = (int)((nx + 63) / 64);
-        const int64_t ntz = (nz + 4 * kSpRZ - 1) / (4 * kSpRZ);
-        hipLaunchKernelGGL(sponge2d_step<kSpRZ>, dim3((unsigned)(ntx * ntz)), dim3(256), 0, stream,
-                           a, ntx);
+        if (reverse && surf.p) {
+            a.surf = surf.p;
+            a.surf_nt = (int)surf_nt;
+        }
+        if (record) a.rec = rec.p;
+        if (sink && sink->dev) {
+            a.snap = sink->dev;
+            a.snap_stride = (int)sink->stride;
+            a.snap_slot0 = sink->slot0;
+        }
+        const int ntx = (int)((nx + kSpCX - 1) / kSpCX);
+        const int64_t ntz = (nz + kSpCZ - 1) / kSpCZ;
+        // 4 rows per wave while the tiles (8 waves each) leave the chip's 1024
+        // SIMDs idle or nearly so, 8 rows from two blocks per CU
+        const dim3 grid((unsigned)(ntx * ntz));
+        if (ntx * ntz < 512)
+            hipLaunchKernelGGL(sponge2d_steps<4>, grid, dim3(64 * kSpZ / 4), 0, stream, a, ntx);
+        else
+            hipLaunchKernelGGL(sponge2d_steps<8>, grid, dim3(64 * kSpZ / 8), 0, stream, a, ntx);
         SSSI_HIP(hipGetLastError());
         cur ^= 1;
     }
@@ -412,12 +556,10 @@ class Prop2D final : public Prop {
             steps_done = done;
             return;
         }
-        for (int64_t q = 0; q < count; ++q) {
-            const int64_t t = reverse ? t_first - q : t_first + q;
-            float *snap = nullptr;
-            if (sink && sink->dev && t % sink->stride == 0)
-                snap = sink->dev + (size_t)(t / sink->stride - sink->slot0) * nz * nx;
-            step_sponge(t, reverse, record, snap, (int)(done + q));
+        for (int64_t q = 0; q < count; q += kSpK) {
+            const int n = (int)std::min<int64_t>(kSpK, count - q);
+            steps_sponge(reverse ? t_first - q : t_first + q, n, reverse, record, sink,
+                         (int)(done + q));
             if (st) st->launches++;
         }
         done += count;
@@ -435,10 +577,10 @@ class Prop2D final : public Prop {
         }, 1 << 16);
     }
 
-    // sponge levels: interior of sp[which], optionally times the second damping factor
+    // sponge levels: interior of the current (0) or old (1) level, optionally times the second damping factor
     void download_sponge(int which, double *out, bool padded_model) {
         std::vector<float> h((size_t)pitch * rows);
-        SSSI_HIP(hipMemcpyAsync(h.data(), sp[which].p, h.size() * sizeof(float),
+        SSSI_HIP(hipMemcpyAsync(h.data(), sp[cur][which].p, h.size() * sizeof(float),
                                 hipMemcpyDeviceToHost, stream));
         SSSI_HIP(hipStreamSynchronize(stream));
         std::vector<float> gf(std::max(nB, 1));
@@ -464,12 +606,12 @@ class Prop2D final : public Prop {
 
     void get_field(double *field) override {
         if (g) g->download((int)(done & 1), field, stream);
-        else download_sponge(cur, field, false);
+        else download_sponge(0, field, false);
     }
 
     void get_model(double *model) override {
         if (!g) {
-            download_sponge(cur ^ 1, model, true);
+            download_sponge(1, model, true);
             return;
         }
         // reference model layout: (nz+2l) x (nx+2l), l-wide zero halo
