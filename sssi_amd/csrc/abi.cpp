@@ -87,7 +87,7 @@ void run_oneshot(Prop &P, int64_t nt, bool reverse, double *data, double *snap, 
         const int64_t per = std::max<int64_t>(1, (int64_t)(256ll << 20) / (cells * 4));
         const int64_t K = std::min(per, nsnap);
         DevBuf<float> stage((size_t)K * cells);
-        HostBuf<float> host((size_t)K * cells);
+        DevBuf<float> turned((size_t)K * cells);
         int64_t done = 0;  // steps executed
         while (done < nt) {
             // slots covered by this chunk
@@ -110,24 +110,9 @@ void run_oneshot(Prop &P, int64_t nt, bool reverse, double *data, double *snap, 
             sink.slot0 = s_lo;
             P.run(t0, count, reverse, data != nullptr, &sink, nullptr);
             const int64_t ns = s_hi - s_lo + 1;
-            SSSI_HIP(hipMemcpyAsync(host.p, stage.p, (size_t)ns * cells * sizeof(float),
-                                    hipMemcpyDeviceToHost, P.stream));
-            SSSI_HIP(hipStreamSynchronize(P.stream));
-            // device slice is x fastest, [z][y][x]: (i*ny + k)*nx + j;
-            // reference layout is z fastest: (k*nx + j)*nz + i.  Split over
-            // host threads by (slice, y, 64-column block); each item writes
-            // whole z columns.
-            const int64_t nz = P.nz, nx = P.nx, ny = P.ny, nxb = (nx + 63) / 64;
-            parallel_ranges(ns * ny * nxb, [&](int64_t a, int64_t b) {
-                for (int64_t it = a; it < b; ++it) {
-                    const int64_t s = it / (ny * nxb), k = (it / nxb) % ny, jb = it % nxb;
-                    const float *src = host.p + s * cells;
-                    double *dst = snap + (s_lo + s) * cells;
-                    for (int64_t j = jb * 64; j < std::min(nx, jb * 64 + 64); ++j)
-                        for (int64_t i = 0; i < nz; ++i)
-                            dst[(k * nx + j) * nz + i] = src[(i * ny + k) * nx + j];
-                }
-            }, 1);
+            // to the reference's layout, z fastest, on the device
+            launch_z_fastest(stage.p, turned.p, P.nz, P.nx, P.ny, ns, P.stream);
+            widen_to_host(snap + s_lo * cells, turned.p, (size_t)ns * cells, P.stream);
             done += count;
         }
     }

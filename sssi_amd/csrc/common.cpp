@@ -5,6 +5,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <system_error>
 
 namespace sssi {
 
@@ -120,6 +121,21 @@ void validate_velocity(const double *v, int64_t n, const char *name) {
              (long long)q, v[q]);
 }
 
+double max_velocity(const double *v, int64_t n) {
+    std::mutex mu;
+    double vmax = 0.0;
+    parallel_ranges(n, [&](int64_t a, int64_t b) {
+        double m[4] = {0.0, 0.0, 0.0, 0.0};  // independent chains
+        int64_t q = a;
+        for (; q + 4 <= b; q += 4)
+            for (int k = 0; k < 4; ++k) m[k] = std::max(m[k], v[q + k]);
+        for (; q < b; ++q) m[0] = std::max(m[0], v[q]);
+        std::lock_guard<std::mutex> lk(mu);
+        vmax = std::max({vmax, m[0], m[1], m[2], m[3]});
+    }, (int64_t)1 << 18);
+    return vmax;
+}
+
 namespace {
 std::mutex g_stream_mu;
 std::map<int, std::vector<hipStream_t>> g_streams;  // idle pool streams per device
@@ -153,6 +169,120 @@ void stream_release(hipStream_t s) {
     }
     std::lock_guard<std::mutex> lk(g_stream_mu);
     g_streams[dev].push_back(s);
+}
+
+namespace {
+// Pinned chunks kept for the next download (hipHostMalloc takes about 0.1 ms
+// per MB): at most kKept of them idle in the process, the rest are freed.
+constexpr size_t kChunkBytes = (size_t)8 << 20;
+constexpr size_t kKept = 4;
+std::mutex g_chunk_mu;
+std::vector<void *> g_chunks;
+
+struct PinnedChunk {
+    void *p = nullptr;
+    PinnedChunk() = default;
+    PinnedChunk(const PinnedChunk &) = delete;
+    PinnedChunk &operator=(const PinnedChunk &) = delete;
+    ~PinnedChunk() {
+        if (!p) return;
+        {
+            std::lock_guard<std::mutex> lk(g_chunk_mu);
+            if (g_chunks.size() < kKept) {
+                g_chunks.push_back(p);
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+    void acquire() {
+        {
+            std::lock_guard<std::mutex> lk(g_chunk_mu);
+            g_chunks.reserve(kKept);  // (giving one back does not allocate)
+            if (!g_chunks.empty()) {
+                p = g_chunks.back();
+                g_chunks.pop_back();
+                return;
+            }
+        }
+        // usable with every device, whichever is current when it is taken again
+        SSSI_HIP(hipHostMalloc(&p, kChunkBytes, hipHostMallocPortable));
+    }
+};
+}  // namespace
+
+void stream_to_host(const void *dev, size_t n, size_t elem, hipStream_t s, const HostUse &use) {
+    if (n == 0) return;
+    const char *src = (const char *)dev;
+    const size_t per = std::max<size_t>(1, kChunkBytes / elem), nchunk = (n + per - 1) / per;
+    PinnedChunk buf[2];
+    buf[0].acquire();
+    if (nchunk > 1) buf[1].acquire();
+    auto fetch = [&](size_t c) {
+        SSSI_HIP(hipMemcpyAsync(buf[c & 1].p, src + c * per * elem,
+                                std::min(per, n - c * per) * elem, hipMemcpyDeviceToHost, s));
+        SSSI_HIP(hipStreamSynchronize(s));
+    };
+    // a worker per MB, up to 15; none for a small result
+    const size_t want = std::min<size_t>({15, n * elem >> 20,
+                                          std::max(1u, std::thread::hardware_concurrency())});
+    std::vector<std::thread> workers;
+    std::atomic<size_t> ready{0}, team{0};
+    std::atomic<bool> stop{false};
+    std::vector<std::atomic<size_t>> done(nchunk);
+    for (auto &d : done) d.store(0);
+    auto work = [&](size_t k) {
+        while (team.load(std::memory_order_acquire) == 0) {
+            if (stop.load(std::memory_order_acquire)) return;
+            std::this_thread::yield();
+        }
+        const size_t T = team.load(std::memory_order_acquire);
+        for (size_t c = 0; c < nchunk; ++c) {
+            while (ready.load(std::memory_order_acquire) <= c) {
+                if (stop.load(std::memory_order_acquire)) return;
+                std::this_thread::yield();
+            }
+            const size_t m = std::min(per, n - c * per), a = m * k / T, b = m * (k + 1) / T;
+            if (b > a) use((const char *)buf[c & 1].p + a * elem, c * per + a, b - a);
+            done[c].fetch_add(1, std::memory_order_release);
+        }
+    };
+    if (want > 1) {
+        workers.reserve(want);
+        try {
+            for (size_t k = 0; k < want; ++k) workers.emplace_back(work, k);
+        } catch (const std::system_error &) {  // no more threads: those there do it
+        }
+    }
+    const size_t T = workers.size();
+    try {
+        if (T > 0) team.store(T, std::memory_order_release);
+        for (size_t c = 0; c < nchunk; ++c) {
+            if (T > 0 && c >= 2)  // the buffer's last chunk has been used
+                while (done[c - 2].load(std::memory_order_acquire) < T) std::this_thread::yield();
+            fetch(c);
+            if (T > 0) ready.store(c + 1, std::memory_order_release);
+            else use(buf[c & 1].p, c * per, std::min(per, n - c * per));
+        }
+    } catch (...) {
+        stop.store(true, std::memory_order_release);
+        for (auto &t : workers) t.join();
+        throw;
+    }
+    for (auto &t : workers) t.join();
+}
+
+void copy_to_host(void *dst, const void *dev, size_t bytes, hipStream_t s) {
+    stream_to_host(dev, bytes, 1, s, [dst](const void *src, size_t first, size_t count) {
+        std::memcpy((char *)dst + first, src, count);
+    });
+}
+
+void widen_to_host(double *dst, const float *dev, size_t n, hipStream_t s) {
+    stream_to_host(dev, n, sizeof(float), s, [dst](const void *src, size_t first, size_t count) {
+        const float *f = (const float *)src;
+        for (size_t q = 0; q < count; ++q) dst[first + q] = f[q];
+    });
 }
 
 }  // namespace sssi

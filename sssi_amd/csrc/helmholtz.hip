@@ -1123,8 +1123,7 @@ struct FreqSystem {
             }
         SSSI_HIP(hipGetLastError());
         SSSI_HIP(hipEventRecord(e1, s));
-        SSSI_HIP(hipMemcpyAsync(U, dU.p, dU.bytes(), hipMemcpyDeviceToHost, s));
-        SSSI_HIP(hipStreamSynchronize(s));
+        copy_to_host(U, dU.p, dU.bytes(), s);
         float ms = 0;
         SSSI_HIP(hipEventElapsedTime(&ms, e0, e1));
         (void)hipEventDestroy(e0);

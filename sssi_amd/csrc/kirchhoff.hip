@@ -545,9 +545,7 @@ class Eikonal2D {
     }
     const double *table() const { return t[cur].p; }
     void download(double *T) {
-        SSSI_HIP(hipMemcpyAsync(T, t[cur].p, (size_t)nz * nx * nsrc * sizeof(double),
-                                hipMemcpyDeviceToHost, stream));
-        SSSI_HIP(hipStreamSynchronize(stream));
+        copy_to_host(T, t[cur].p, (size_t)nz * nx * nsrc * sizeof(double), stream);
     }
 };
 

@@ -45,6 +45,10 @@ struct SnapSink {
     int64_t slot0 = 0;
 };
 
+// Snapshot slices (x fastest, [s][z][y][x]) to z fastest ([s][y][x][z]).
+void launch_z_fastest(const float *in, float *out, int64_t nz, int64_t nx, int64_t ny, int64_t ns,
+                      hipStream_t s);
+
 class Prop {
    public:
     // the stream is destroyed here, so that a derived constructor that throws

@@ -251,6 +251,39 @@ __global__ void __launch_bounds__(64 * kSpZ / R) sponge2d_steps(Sponge2dArgs a, 
         sponge2d_tile<R, false>(a, tx, ty, edge);
 }
 
+// One (slice, y) plane's 64 x 64 tile through LDS: rows of x in, columns of z
+// out, both coalesced; 65 floats per LDS row keep the banks apart.
+__global__ void __launch_bounds__(256) z_fastest(const float *__restrict__ in,
+                                                 float *__restrict__ out, int64_t nz, int64_t nx,
+                                                 int64_t ny, int64_t ntx, int64_t ntz,
+                                                 int64_t ntiles) {
+    __shared__ float t[64][65];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int64_t b = blockIdx.x; b < ntiles; b += gridDim.x) {
+        const int64_t x0 = b % ntx * 64, z0 = b / ntx % ntz * 64, sy = b / (ntx * ntz);
+        const int64_t y = sy % ny, base = sy / ny * (nz * nx * ny);
+#pragma unroll 4
+        for (int r = w; r < 64; r += 4)
+            if (z0 + r < nz && x0 + lane < nx)
+                t[r][lane] = in[base + ((z0 + r) * ny + y) * nx + x0 + lane];
+        __syncthreads();
+#pragma unroll 4
+        for (int r = w; r < 64; r += 4)
+            if (x0 + r < nx && z0 + lane < nz)
+                out[base + (y * nx + x0 + r) * nz + z0 + lane] = t[lane][r];
+        __syncthreads();
+    }
+}
+
+void launch_z_fastest(const float *in, float *out, int64_t nz, int64_t nx, int64_t ny, int64_t ns,
+                      hipStream_t s) {
+    const int64_t ntx = (nx + 63) / 64, ntz = (nz + 63) / 64, n = ntx * ntz * ny * ns;
+    if (n == 0) return;
+    hipLaunchKernelGGL(z_fastest, dim3((unsigned)std::min<int64_t>(n, 1 << 20)), dim3(256), 0, s,
+                       in, out, nz, nx, ny, ntx, ntz, n);
+    SSSI_HIP(hipGetLastError());
+}
+
 // ---------------------------------------------------------------------------
 class Prop2D final : public Prop {
    public:
@@ -276,8 +309,7 @@ class Prop2D final : public Prop {
         SSSI_HIP(hipGetDevice(&device));
         stream = stream_acquire();
         {
-            double vmax = 0.0;
-            for (int64_t q = 0; q < nz * nx; ++q) vmax = std::max(vmax, v[q]);
+            const double vmax = max_velocity(v, nz * nx);
             courant = vmax * dt * std::sqrt(1.0 / (dz * dz) + 1.0 / (dx * dx));
         }
         if (abc == SSSI_ABC_CPML) {
@@ -569,12 +601,7 @@ class Prop2D final : public Prop {
     void get_data(double *data, int64_t nt) override {
         if (nt > rec_nt || !rec.p)
             fail(SSSI_ESTATE, "get_data: no recorded traces for %lld steps", (long long)nt);
-        HostBuf<float> h((size_t)nt * nx);
-        SSSI_HIP(hipMemcpyAsync(h.p, rec.p, h.bytes(), hipMemcpyDeviceToHost, stream));
-        SSSI_HIP(hipStreamSynchronize(stream));
-        parallel_ranges((int64_t)h.n, [&](int64_t a, int64_t b) {
-            for (int64_t q = a; q < b; ++q) data[q] = h.p[q];  // [t][j] == data(nx,nt)
-        }, 1 << 16);
+        widen_to_host(data, rec.p, (size_t)nt * nx, stream);  // [t][j] == data(nx,nt)
     }
 
     // sponge levels: interior of the current (0) or old (1) level, optionally times the second damping factor

@@ -783,8 +783,7 @@ class Prop3D final : public Prop {
         SSSI_HIP(hipGetDevice(&device));
         stream = stream_acquire();
         {
-            double vmax = 0.0;
-            for (int64_t q = 0; q < nz * nx * ny; ++q) vmax = std::max(vmax, v[q]);
+            const double vmax = max_velocity(v, nz * nx * ny);
             courant = vmax * dt * std::sqrt(1.0 / (dz * dz) + 1.0 / (dx * dx) + 1.0 / (dy * dy));
         }
         health.alloc(1);
@@ -1201,12 +1200,7 @@ class Prop3D final : public Prop {
 
     void get_data(double *data, int64_t nt) override {
         if (nt > rec_nt || !rec.p) fail(SSSI_ESTATE, "get_data: no recorded traces");
-        HostBuf<float> h((size_t)nt * nx * ny);
-        SSSI_HIP(hipMemcpyAsync(h.p, rec.p, h.bytes(), hipMemcpyDeviceToHost, stream));
-        SSSI_HIP(hipStreamSynchronize(stream));
-        parallel_ranges((int64_t)h.n, [&](int64_t a, int64_t b) {
-            for (int64_t q = a; q < b; ++q) data[q] = h.p[q];  // [t][k][j] == data(nx,ny,nt)
-        }, 1 << 16);
+        widen_to_host(data, rec.p, (size_t)nt * nx * ny, stream);  // [t][k][j] == data(nx,ny,nt)
     }
 
     void get_field(double *field) override {

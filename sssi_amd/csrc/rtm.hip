@@ -598,9 +598,7 @@ int sssi_rtm2d_get_stack(sssi_rtm *r, double *stack) {
     return rtm_guard([&] {
         if (!stack) fail(SSSI_EINVAL, "stack must not be NULL");
         Rtm2D &rt = R(r);
-        SSSI_HIP(hipMemcpyAsync(stack, rt.stack.p, rt.stack.bytes(), hipMemcpyDeviceToHost,
-                                rt.stream));
-        SSSI_HIP(hipStreamSynchronize(rt.stream));
+        copy_to_host(stack, rt.stack.p, rt.stack.bytes(), rt.stream);
     });
 }
 
