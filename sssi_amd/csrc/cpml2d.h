@@ -139,6 +139,20 @@ void launch_cpml2d_single(const Cpml2dGrid &g, const Job2D &job, const int2 *ord
                           int step, hipStream_t s, const int *base = nullptr);
 void launch_cpml2d_single(int N, int rz, int ng, const Job2D &job, const int2 *order, int nblk,
                           int step, hipStream_t s, const int *base = nullptr);
+// Several steps per launch on small grids (cpml2d_steps): most steps of one
+// launch for the grid, 0 where a launch per step is as good (or SSSI_STEPS=0,
+// or SSSI_NG / SSSI_RZ name a layout of the step kernel).
+int cpml2d_steps_per_launch(const Cpml2dGrid &g);
+constexpr int kStepsMaxSrc = 64;  // most point sources of a job it takes
+// Where such a launch writes: levels current and old after its last step, and
+// the memory variables; none of them is an input of the launch.
+struct Steps2DOut {
+    float *p, *pold, *zphi, *zpsi, *xphi, *xpsi;
+};
+// n <= cpml2d_steps_per_launch steps of a job without checkpoints and imaging,
+// from launch step `step` on.
+void launch_cpml2d_steps(const Cpml2dGrid &g, const Job2D &job, const Steps2DOut &out, int step,
+                         int n, hipStream_t s);
 // Launch one step of many jobs sharing nDiffOrder, rz and march layout
 // (descriptors in device memory).
 void launch_cpml2d_batch(int N, int rz, int ng, const Job2D *jobs, const int2 *order, int nblk,

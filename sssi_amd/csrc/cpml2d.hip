@@ -27,6 +27,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <numeric>
+#include <type_traits>
 
 #include "cpml2d.h"
 #include "devbuf.h"
@@ -726,6 +727,330 @@ __global__ void step_base_add(int *base, int k) {
     if (threadIdx.x == 0) *base += k;
 }
 
+// Several time steps per launch, for grids on which a step's launch and load
+// latency take longer than its work.  A workgroup holds an EZ x 64 tile (lane =
+// column, R rows per wavefront): p in LDS (two buffers), the previous level,
+// v^2 dt^2 and the memory variables of its cells in registers.  Each step is
+// the step kernel's arithmetic cell by cell -- the same stencil form for a
+// cell as the 64 x rz tile it lies in takes there -- with A_x and A_z of the
+// damping strips through LDS.  Cells within L of the tile's edge miss
+// neighbours and go wrong, and each step moves that error L cells inwards, so
+// after n <= K steps the inner CZ x CX cells are exact and are what the tile
+// writes, into buffers other than those its neighbours still read.  Cells
+// outside the model stay 0, which is the boundary.
+// Bound by vector issue: the step kernel takes ~7 us per step on these grids
+// whatever their size, this one ~5 us per launch and then ~1.2 us (N = 1) to
+// ~3 us (N = 4) per step and round of workgroups.  120 x 240 cells, 600 steps,
+// whole call, one step per launch -> this kernel: N=1 4.08 -> 1.37 ms, N=2 4.08
+// -> 2.00, N=3 4.20 -> 3.29, N=4 4.31 -> 3.54; 300 x 500 cells: N=1 4.23 ->
+// 1.62, N=2 4.34 -> 2.77, N=3 4.37 -> 3.74.  K and W are the best of a sweep
+// there (N=2: K=4 with 12 waves 2.43, K=3 with 8 waves 2.52, K=5 with 9 waves
+// 2.30 ms): a larger tile wastes less of itself on its rim but gives fewer
+// workgroups, with more waves to a SIMD.  For N >= 5 the rim (18 cells at K=2)
+// is most of the tile and one step per launch is faster (N=5: 4.55 vs 5.68).
+template <int N>
+struct Steps2D {
+    static constexpr int L = 2 * N - 1;
+    static constexpr int K = N == 1 ? 8 : N == 2 ? 4 : N == 3 ? 3 : 2;
+    static constexpr int R = 4, W = N == 3 ? 12 : 8;
+    static constexpr int EZ = R * W, H = K * L, CX = kTX - 2 * H, CZ = EZ - 2 * H;
+};
+
+template <int N>
+__global__ void __launch_bounds__(64 * Steps2D<N>::W) cpml2d_steps(Job2D J, Steps2DOut O, int rz,
+                                                                   int ntx, int step0, int n) {
+    using T = Steps2D<N>;
+    constexpr int L = T::L, R = T::R, EZ = T::EZ, H = T::H, PAD = 16;
+    // L (s_az: N) rows of zeros above and below the tile, so that a wave's
+    // windows need no clamp: one base and constant offsets
+    __shared__ float s_p[2][(EZ + 2 * L) * kTX + 2 * PAD], s_ax[EZ * kTX + 2 * PAD],
+        s_az[(EZ + 2 * N) * kTX];
+    const int lane = threadIdx.x & 63, w = wave_id();
+    const int ty = (int)blockIdx.x / ntx, tx = (int)blockIdx.x - ty * ntx;
+    const int nz = J.nz, nx = J.nx, nB = J.nB, nb2 = 2 * nB, zb0 = nz - nB;
+    const int j = tx * T::CX - H + lane;
+    const int q0 = w * R, i0 = ty * T::CZ - H + q0;  // the wave's first row: in the tile, in the model
+    const bool jin = j >= 0 && j < nx;
+    const bool jmine = jin && lane >= H && lane < kTX - H;
+    auto iin = [&](int r) { return i0 + r >= 0 && i0 + r < nz; };
+    auto mine = [&](int r) { return iin(r) && q0 + r >= H && q0 + r < EZ - H; };
+    const int rel0 = step0 - J.start_step, par = rel0 & 1;
+    const uint32_t rowb = (uint32_t)J.pitch * 4u, nbytes = rowb * (uint32_t)J.rows;
+    const uint32_t vcol = jin ? (uint32_t)(j + kHX) * 4u : kOOB;
+    auto srow = [&](int r) { return (uint32_t)(i0 + r + kHZ) * rowb; };
+
+    // which form a cell takes: its 64 x rz tile within reach of an x / z strip
+    const int xt = (j < 0 ? 0 : j) / kTX * kTX;
+    const bool xs = nB > 0 && (xt - N < nB || xt + kTX + N - 1 > nx - nB);
+    auto zstrip = [&](int i) { return nB > 0 && i >= 0 && i / rz * rz + rz + N - 1 > zb0; };
+    const bool xblock = __ballot(jin && xs) != 0;
+    const bool zblock = zstrip(min(ty * T::CZ - H + EZ - 1, nz - 1));
+    // own cell in a strip: byte offset, kOOB where there is none
+    const bool xown = jin && (j < nB || j >= nx - nB);
+    const uint32_t xcol = xown ? (uint32_t)(j < nB ? j : j - (nx - nb2)) * 4u : kOOB;
+    auto xoff = [&](int r) { return iin(r) ? xcol + (uint32_t)(i0 + r) * (uint32_t)nb2 * 4u : kOOB; };
+    auto zown = [&](int r) { return nB > 0 && i0 + r >= zb0 && i0 + r < nz; };
+    auto zoff = [&](int r) {
+        return zown(r) && jin ? (uint32_t)(i0 + r - zb0) * (uint32_t)nx * 4u + (uint32_t)j * 4u : kOOB;
+    };
+
+    float p[R], po[R], v2[R], xph[R], xps[R], xb[R], zph[R], zps[R], zb[R];
+    int keep[R];
+    {
+        const __amdgpu_buffer_rsrc_t rP = buf_rsrc(J.p[par], nbytes);
+        const __amdgpu_buffer_rsrc_t rO = buf_rsrc(J.p[par ^ 1], nbytes);
+        const __amdgpu_buffer_rsrc_t rV = buf_rsrc(J.vdt2, nbytes);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t v = iin(r) ? vcol : kOOB, so = iin(r) ? srow(r) : 0u;
+            p[r] = buf_ld(rP, v, so);
+            po[r] = buf_ld(rO, v, so);
+            v2[r] = buf_ld(rV, v, so);
+            keep[r] = jin && iin(r) ? -1 : 0;
+            xph[r] = xps[r] = xb[r] = zph[r] = zps[r] = zb[r] = 0.f;
+        }
+    }
+    if (xblock) {
+        const uint32_t nb = (uint32_t)nz * (uint32_t)nb2 * 4u;
+        const __amdgpu_buffer_rsrc_t a = buf_rsrc(J.xphi[par], nb), b = buf_rsrc(J.xpsi, nb),
+                                     c = buf_rsrc(J.xbm1, nb);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t o = xoff(r);
+            xph[r] = buf_ld(a, o, 0);
+            xps[r] = buf_ld(b, o, 0);
+            xb[r] = buf_ld(c, o, 0);
+        }
+    }
+    if (zblock) {
+        const uint32_t nb = (uint32_t)nB * (uint32_t)nx * 4u;
+        const __amdgpu_buffer_rsrc_t a = buf_rsrc(J.zphi[par], nb), b = buf_rsrc(J.zpsi, nb),
+                                     c = buf_rsrc(J.zbm1, nb);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t o = zoff(r);
+            zph[r] = buf_ld(a, o, 0);
+            zps[r] = buf_ld(b, o, 0);
+            zb[r] = buf_ld(c, o, 0);
+        }
+    }
+    // sources among the wave's cells
+    bool has_src = false;
+    if (!J.reverse && J.src_ptr)
+        for (int k = 0; k < J.nsrc; ++k) {
+            const int cell = ld_uniform(J.src_cell + k), ci = cell / nx, cj = cell - ci * nx;
+            has_src |= ci >= i0 && ci < i0 + R && cj >= tx * T::CX - H && cj < tx * T::CX - H + kTX;
+        }
+    const bool top = i0 <= 0 && i0 + R > 0;  // the wave holds row 0
+    const bool surf_here = top && J.reverse && J.surf;
+
+#pragma unroll
+    for (int r = 0; r < R; ++r) s_p[0][PAD + (L + q0 + r) * kTX + lane] = p[r];
+    for (int r = w; r < 2 * L; r += T::W) {
+        const int o = PAD + (r < L ? r : EZ + r) * kTX + lane;
+        s_p[0][o] = s_p[1][o] = 0.f;
+    }
+    for (int r = w; r < 2 * N; r += T::W) s_az[(r < N ? r : EZ + r) * kTX + lane] = 0.f;
+    __syncthreads();
+    // row flags as lane masks: rows that take the two-stage z form, rows in the strip
+    int zsm[R], zom[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        zsm[r] = zblock && zstrip(i0 + r) ? -1 : 0;
+        zom[r] = zown(r) ? -1 : 0;
+    }
+    auto pick = [](int m, float x, float y) {  // m ? x : y without a branch
+        return __int_as_float((__float_as_int(x) & m) | (__float_as_int(y) & ~m));
+    };
+    const int xsm = xs ? -1 : 0, xom = xown ? -1 : 0;
+
+    // the steps, compiled per kind of strip in the tile's reach (each row's
+    // work is then free of branches, and the rows overlap)
+    auto steps = [&](auto XB, auto ZB) {
+#pragma unroll 1
+        for (int s = 0; s < n; ++s) {
+            const int t = J.reverse ? J.nt - 1 - (rel0 + s) : rel0 + s;
+            const float *P = s_p[s & 1] + PAD + (L + q0) * kTX + lane;
+            // z window: rows q0-L .. q0+R-1+L of the lane's column
+            float col[R + 2 * L];
+#pragma unroll
+            for (int r = 0; r < L; ++r) {
+                col[r] = P[(r - L) * kTX];
+                col[L + R + r] = P[(R + r) * kTX];
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r) col[L + r] = p[r];
+            float lap[R];
+            if constexpr (!XB && !ZB) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float *row = P + r * kTX;
+                    float acc = J.w0 * col[L + r];
+#pragma unroll
+                    for (int m = 1; m <= L; ++m)
+                        acc = fmaf(J.wz[m], col[L + r + m] + col[L + r - m], acc);
+#pragma unroll
+                    for (int m = 1; m <= L; ++m) acc = fmaf(J.wx[m], row[m] + row[-m], acc);
+                    lap[r] = fmaf(J.w0lo, col[L + r], acc);
+                }
+            } else {
+                // A at the half points of the own cells, through LDS (off a
+                // strip b-1 = Phi = 0 and A = D)
+                if constexpr (ZB) {
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        float d = 0.f;
+#pragma unroll
+                        for (int k = 0; k < N; ++k)
+                            d = fmaf(J.cz[k], col[L + r + 1 + k] - col[L + r - k], d);
+                        zph[r] = fmaf(zb[r], zph[r] + d, zph[r]);
+                        s_az[(N + q0 + r) * kTX + lane] = pick(zom[r], d + zph[r], d);
+                    }
+                }
+                if constexpr (XB) {
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const float *row = P + r * kTX;
+                        float d = 0.f;
+#pragma unroll
+                        for (int k = 0; k < N; ++k) d = fmaf(J.cx[k], row[1 + k] - row[-k], d);
+                        xph[r] = fmaf(xb[r], xph[r] + d, xph[r]);
+                        s_ax[PAD + (q0 + r) * kTX + lane] = pick(xom, d + xph[r], d);
+                    }
+                }
+                // the composite forms: z alone, x alone, both as one sum
+                float dz[R], dx[R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const float *row = P + r * kTX;
+                    float az = J.w0z * col[L + r], ax = J.w0x * col[L + r], all = J.w0 * col[L + r];
+#pragma unroll
+                    for (int m = 1; m <= L; ++m) {
+                        const float zz = col[L + r + m] + col[L + r - m];
+                        if constexpr (XB) az = fmaf(J.wz[m], zz, az);
+                        all = fmaf(J.wz[m], zz, all);
+                    }
+#pragma unroll
+                    for (int m = 1; m <= L; ++m) {
+                        const float xx = row[m] + row[-m];
+                        if constexpr (ZB) ax = fmaf(J.wx[m], xx, ax);
+                        all = fmaf(J.wx[m], xx, all);
+                    }
+                    dz[r] = fmaf(J.w0zlo, col[L + r], az);
+                    dx[r] = fmaf(J.w0xlo, col[L + r], ax);
+                    lap[r] = fmaf(J.w0lo, col[L + r], all);
+                }
+                __syncthreads();
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    if constexpr (ZB) {
+                        const float *a = s_az + (N + q0 + r) * kTX + lane;
+                        float d = 0.f;
+#pragma unroll
+                        for (int k = 0; k < N; ++k)
+                            d = fmaf(J.cz[k], a[k * kTX] - a[-(1 + k) * kTX], d);
+                        zps[r] = fmaf(zb[r], zps[r] + d, zps[r]);
+                        dz[r] = pick(zsm[r], pick(zom[r], d + zps[r], d), dz[r]);
+                    }
+                    if constexpr (XB) {
+                        const float *a = s_ax + PAD + (q0 + r) * kTX + lane;
+                        float d = 0.f;
+#pragma unroll
+                        for (int k = 0; k < N; ++k) d = fmaf(J.cx[k], a[k] - a[-1 - k], d);
+                        xps[r] = fmaf(xb[r], xps[r] + d, xps[r]);
+                        dx[r] = pick(xsm, pick(xom, d + xps[r], d), dx[r]);
+                    }
+                    lap[r] = pick(zsm[r] | (XB ? xsm : 0), dz[r] + dx[r], lap[r]);
+                }
+            }
+            if (has_src || surf_here) {  // wave-uniform
+                float sv[R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) sv[r] = 0.f;
+                if (has_src && t < J.src_nt)
+                    for (int k = 0; k < J.nsrc; ++k) {
+                        const int cell = ld_uniform(J.src_cell + k), ci = cell / nx, cj = cell - ci * nx;
+                        const float a = ld_uniform(J.src_amp + (size_t)t * J.nsrc + k);
+                        if (cj == j) {
+#pragma unroll
+                            for (int r = 0; r < R; ++r)
+                                if (ci == i0 + r) sv[r] += a;
+                        }
+                    }
+                if (surf_here && t < J.surf_nt && jin) {
+                    const size_t o = (size_t)t * nx + j;
+                    const float x = J.surf2 ? J.surf[o] - J.surf2[o] : J.surf[o];
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (i0 + r == 0) sv[r] += x;
+                }
+#pragma unroll
+                for (int r = 0; r < R; ++r) lap[r] += sv[r];
+            }
+            float *Q = s_p[(s & 1) ^ 1] + PAD + (L + q0) * kTX + lane;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const float pn = p[r] + fmaf(v2[r], lap[r], p[r] - po[r]);
+                po[r] = p[r];
+                p[r] = __int_as_float(__float_as_int(pn) & keep[r]);
+                Q[r * kTX] = p[r];
+            }
+            if (top) {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (i0 + r == 0 && mine(r)) {
+                        if (J.rec && jmine) J.rec[(size_t)t * nx + j] = p[r];
+                        if (J.health) report_nonfinite(J.health, jmine && nonfinite(p[r]), step0 + s);
+                    }
+            }
+            if (J.snap && t % J.snap_stride == 0) {
+                const __amdgpu_buffer_rsrc_t rS = buf_rsrc(
+                    J.snap + (size_t)(t / J.snap_stride - J.snap_slot0) * nz * nx,
+                    (uint32_t)nz * (uint32_t)nx * 4u);
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    buf_st(p[r], rS, mine(r) && jmine ? (uint32_t)j * 4u : kOOB,
+                           mine(r) ? (uint32_t)(i0 + r) * (uint32_t)nx * 4u : 0u);
+            }
+            __syncthreads();
+        }
+    };
+    using Y = std::true_type;
+    using F = std::false_type;
+    if (xblock && zblock) steps(Y{}, Y{});
+    else if (xblock) steps(Y{}, F{});
+    else if (zblock) steps(F{}, Y{});
+    else steps(F{}, F{});
+
+    const __amdgpu_buffer_rsrc_t wP = buf_rsrc(O.p, nbytes), wO = buf_rsrc(O.pold, nbytes);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t v = mine(r) && jmine ? vcol : kOOB, so = mine(r) ? srow(r) : 0u;
+        buf_st(p[r], wP, v, so);
+        buf_st(po[r], wO, v, so);
+    }
+    if (xblock) {
+        const uint32_t nb = (uint32_t)nz * (uint32_t)nb2 * 4u;
+        const __amdgpu_buffer_rsrc_t a = buf_rsrc(O.xphi, nb), b = buf_rsrc(O.xpsi, nb);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t o = mine(r) && jmine ? xoff(r) : kOOB;
+            buf_st(xph[r], a, o, 0);
+            buf_st(xps[r], b, o, 0);
+        }
+    }
+    if (zblock) {
+        const uint32_t nb = (uint32_t)nB * (uint32_t)nx * 4u;
+        const __amdgpu_buffer_rsrc_t a = buf_rsrc(O.zphi, nb), b = buf_rsrc(O.zpsi, nb);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t o = mine(r) && jmine ? zoff(r) : kOOB;
+            buf_st(zph[r], a, o, 0);
+            buf_st(zps[r], b, o, 0);
+        }
+    }
+}
+
 // Pack a staged FP32 checkpoint into 16 bits after the job's last step.
 __global__ void ck_pack(float *stage, uint16_t *out, const unsigned *mx, float *scale_out,
                         size_t n, int fmt) {
@@ -1105,6 +1430,53 @@ void launch_cpml2d_batch(int N, int rz, int ng, const Job2D *jobs, const int2 *o
                        base)
     SSSI_NRZ_SWITCH(N, rz, ng, SSSI_LB)
 #undef SSSI_LB
+    SSSI_HIP(hipGetLastError());
+}
+
+// The several-step kernel is taken up to the tile count at which its rounds of
+// workgroups cost what it saves in launches.  Whole calls of 600 steps, one step
+// per launch vs several, ms: N=1 1100 tiles (700 x 1200) 5.33 vs 4.29, 1824
+// tiles 5.83 vs 6.39; N=2 645 tiles (340 x 600) 4.37 vs 3.50, 850 tiles 4.55 vs
+// 4.64; N=3 255 tiles (300 x 500) 4.30 vs 3.75, 306 tiles 4.39 vs 5.09; N=4 240
+// tiles (118 x 270) 4.33 vs 3.48, 264 tiles 4.85 vs 6.00 (here and at N=3 a CU
+// holds one workgroup, and the 257th starts a second round).
+template <int N>
+static int steps_rule(const Cpml2dGrid &g) {
+    using T = Steps2D<N>;
+    constexpr int64_t limit = N == 1 ? 1024 : N == 2 ? 640 : 256;
+    const int64_t tiles = ((g.nx + T::CX - 1) / T::CX) * ((g.nz + T::CZ - 1) / T::CZ);
+    return tiles <= limit ? T::K : 0;
+}
+
+// SSSI_STEPS=0: one step per launch everywhere (as with SSSI_NG / SSSI_RZ, which
+// choose a layout of the step kernel).
+int cpml2d_steps_per_launch(const Cpml2dGrid &g) {
+    if (env_int("SSSI_STEPS", 1) == 0 || std::getenv("SSSI_NG") || std::getenv("SSSI_RZ")) return 0;
+    switch (g.N) {
+        case 1: return steps_rule<1>(g);
+        case 2: return steps_rule<2>(g);
+        case 3: return steps_rule<3>(g);
+        case 4: return steps_rule<4>(g);
+        default: return 0;
+    }
+}
+
+void launch_cpml2d_steps(const Cpml2dGrid &g, const Job2D &job, const Steps2DOut &out, int step,
+                         int n, hipStream_t s) {
+#define SSSI_LS(NN)                                                                           \
+    case NN: {                                                                                \
+        using T = Steps2D<NN>;                                                                \
+        const int ntx = (int)((g.nx + T::CX - 1) / T::CX);                                    \
+        const int ntz = (int)((g.nz + T::CZ - 1) / T::CZ);                                    \
+        hipLaunchKernelGGL(cpml2d_steps<NN>, dim3((unsigned)(ntx * ntz)), dim3(64 * T::W), 0, \
+                           s, job, out, g.rz, ntx, step, n);                                  \
+        break;                                                                                \
+    }
+    switch (g.N) {
+        SSSI_LS(1) SSSI_LS(2) SSSI_LS(3) SSSI_LS(4)
+        default: fail(SSSI_EINVAL, "no several-step kernel for nDiffOrder=%d", g.N);
+    }
+#undef SSSI_LS
     SSSI_HIP(hipGetLastError());
 }
 

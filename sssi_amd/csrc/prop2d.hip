@@ -292,6 +292,9 @@ class Prop2D final : public Prop {
     DevSources srcs;
     DevBuf<int2> order;
     int nblk = 0;
+    // second set of levels and memory variables (several steps per launch:
+    // a launch reads one set and writes the other)
+    DevBuf<float> ap[2], azpsi, axpsi;
     StepGraph graph;   // captured time loop (re-captured when the descriptor changes)
     int64_t done = 0;  // steps since reset (parity of the current level)
     // sponge
@@ -576,6 +579,12 @@ class Prop2D final : public Prop {
         if (count < 0) fail(SSSI_EINVAL, "run: negative step count");
         if (count == 0) return;
         if (record) ensure_rec(reverse ? t_first + 1 : t_first + count, nx);
+        const int K = g && count > 1 && !graphs_enabled() && srcs.n <= kStepsMaxSrc
+                          ? cpml2d_steps_per_launch(*g) : 0;
+        if (K > 0) {
+            run_steps(t_first, count, reverse, record, sink, K, st);
+            return;
+        }
         if (g) {
             int step0;
             const Job2D J = make_job(t_first, reverse, record, sink, &step0);
@@ -595,6 +604,44 @@ class Prop2D final : public Prop {
             if (st) st->launches++;
         }
         done += count;
+        steps_done = done;
+    }
+
+    // Up to K steps per launch.  The grid's buffers are swapped with the second
+    // set so that the present levels and memory variables stay where make_job,
+    // get_field and get_model look for them (by the parity of `done`).
+    void run_steps(int64_t t_first, int64_t count, bool reverse, bool record,
+                   const SnapSink *sink, int K, LaunchStats *st) {
+        if (!ap[0].p) {
+            for (auto &b : ap) {
+                b.alloc(g->p[0].n);
+                SSSI_HIP(hipMemsetAsync(b.p, 0, b.bytes(), stream));  // (its padding stays 0)
+            }
+            if (nB > 0) {
+                azpsi.alloc(g->zpsi.n);
+                axpsi.alloc(g->xpsi.n);
+            }
+        }
+        for (int64_t q = 0; q < count;) {
+            const int n = (int)std::min<int64_t>(K, count - q);
+            int step;
+            const Job2D J = make_job(reverse ? t_first - q : t_first + q, reverse, record, sink, &step);
+            const int lev = (int)(done & 1), to = (int)((done + n) & 1);
+            const Steps2DOut out{ap[0].p, ap[1].p, g->zphi[lev ^ 1].p, azpsi.p, g->xphi[lev ^ 1].p,
+                                 axpsi.p};
+            launch_cpml2d_steps(*g, J, out, step, n, stream);
+            if (st) st->launches++;
+            std::swap(g->p[to], ap[0]);
+            std::swap(g->p[to ^ 1], ap[1]);
+            std::swap(g->zpsi, azpsi);
+            std::swap(g->xpsi, axpsi);
+            if (to == lev) {  // the new Phi lies where the other parity's belongs
+                std::swap(g->zphi[0], g->zphi[1]);
+                std::swap(g->xphi[0], g->xphi[1]);
+            }
+            done += n;
+            q += n;
+        }
         steps_done = done;
     }
 
