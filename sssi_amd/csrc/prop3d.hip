@@ -793,6 +793,7 @@ class Prop3D final : public Prop {
         }
         if (const char *e = std::getenv("SSSI_PD3")) pd_override = std::atoi(e);
         if (const char *e = std::getenv("SSSI_RING3")) ring_on = std::atoi(e) != 0;
+        zc = default_chunk();
         if (const char *e = std::getenv("SSSI_ZC3")) {
             const int z = std::atoi(e);
             if (z >= 8 && z <= 4096) zc = z;
@@ -1054,6 +1055,21 @@ class Prop3D final : public Prop {
             }
         }
         launch_pd<NN, TY, 2>(args, nblk);
+    }
+
+    // Planes per z chunk.  A block reads and starts up on planes outside its chunk, which
+    // long chunks pay less often, but a grid of few chunks leaves CUs idle.
+    // us per step (order 4 unless named) at chunks of 8 / 16 / 24 / 32 planes:
+    // 160 blocks of 32 planes (300 x 100 x 64, order 3) 38.6 / 48.8 / 54.8 / 69.8;
+    // 240 (100 x 200 x 120, order 5) 73 / 78 / 91 / 93; 270 (130 x 140 x 140) 68 /
+    // 78 / 85 / 96; 300 (160^3) 56 / 56 / 62 / 79; 432 (180 x 190 x 190) 71 / 74 / 66 /
+    // 81; 600 (170 x 250 x 200) 84 / 76 / 80 / 84; 700 (200^3, order 2) 86 / 87 / 89 /
+    // 84; 784 (220 x 250 x 220) 113 / 104 / 103 / 105; 5390 (420 x 440 x 440)
+    // 591 / 529 / 504 / 490.
+    int default_chunk() const {
+        const int64_t blocks =
+            ((nx + kTX - 1) / kTX) * ((ny + ty - 1) / ty) * ((nz + 31) / 32);
+        return blocks <= 384 ? 8 : blocks <= 640 ? 24 : 32;
     }
 
     // z split of the sweep: chunks above zsplit never reach the bottom strip
