@@ -108,8 +108,8 @@ __device__ __forceinline__ double wave_shl1(double v) {
 // The passes are bound by FP64 issue, so what pays is running fewer of them:
 // only a band around the front and the places it comes back to can change.
 // A call for 64 tables of 300 x 600 (1800 passes) took 67.1 ms with every
-// tile run and takes 20.5 ms; one table of 101 x 151 (504 passes) 1.25 and
-// 0.87 ms.
+// tile run and takes 20.5 ms (14.4 since the tables come to the host in pinned
+// chunks); one table of 101 x 151 (504 passes) 1.25 and 0.87 ms.
 struct EikList {
     const int *list;   // this launch's tiles, or null: all of them
     const int *count;  // their number (list given)
