@@ -109,7 +109,8 @@ __device__ __forceinline__ double wave_shl1(double v) {
 // only a band around the front and the places it comes back to can change.
 // A call for 64 tables of 300 x 600 (1800 passes) took 67.1 ms with every
 // tile run and takes 20.5 ms (14.4 since the tables come to the host in pinned
-// chunks); one table of 101 x 151 (504 passes) 1.25 and 0.87 ms.
+// chunks); one table of 101 x 151 (504 passes) 1.25 and 0.87 ms (0.52 on the
+// narrow tiles of EikLayout).
 struct EikList {
     const int *list;   // this launch's tiles, or null: all of them
     const int *count;  // their number (list given)
@@ -407,11 +408,19 @@ constexpr int kShotGroup = 8;  // most shots per workgroup row of kirch_group
 constexpr int64_t kEikBlocks = 2560;
 
 // Pass kernel choice: H passes per launch on 64 x TW tiles, or (h = 0) the
-// plain one-pass kernel.  SSSI_EIK = "plain" | "<H>x<TW>" (4x32, 4x64, 8x48,
-// 8x64) overrides the default 4x32.  Cell-passes per second on 600 tables of
+// plain one-pass kernel.  SSSI_EIK = "plain" | "<H>x<TW>" (4x32, 4x64, 8x24, 8x48,
+// 8x64) overrides the default.  Cell-passes per second on 600 tables of
 // a 300 x 600 grid, 1800 passes, every tile run: plain 148 G, 4x32 369 G, 8x48 315 G,
 // 4x64 273 G, 8x64 261 G (the wider tiles hold 16 columns per wave in
-// registers, 176+ VGPRs, and run 2 waves per SIMD).
+// registers, 176+ VGPRs, and run 2 waves per SIMD).  Where a launch's list holds
+// fewer tiles than the chip has CUs, a pass takes as long as its FP64 issue on
+// one tile, and narrow tiles (6 columns per wave) and half the launches are
+// faster although the tiles compute 4 times the cells they write: whole calls,
+// 4x32 -> 8x24, 101 x 151 (504 passes) 0.90 -> 0.52 ms for one table, 1.06 -> 0.69
+// for 8, 1.52 -> 1.29 for 32; 300 x 600 (1800 passes) 3.13 -> 1.85 for one, 3.96
+// -> 2.80 for 4, 6.45 -> 5.50 for 16; 14.4 -> 15.1 for 64, where every CU has work
+// and the recomputed cells count.  So 8x24 up to 3e6 cells over all tables.
+constexpr double kEikNarrowCells = 3e6;
 struct EikLayout {
     int h = 4, tw = 32;
     void launch(dim3 grid, hipStream_t s, const double *slow, const double *told, double *tnew,
@@ -425,6 +434,7 @@ struct EikLayout {
     }
         SSSI_EIK_CASE(4, 32)
         SSSI_EIK_CASE(4, 64)
+        SSSI_EIK_CASE(8, 24)
         SSSI_EIK_CASE(8, 48)
         SSSI_EIK_CASE(8, 64)
 #undef SSSI_EIK_CASE
@@ -432,8 +442,9 @@ struct EikLayout {
     }
 };
 
-static EikLayout eik_layout() {
+static EikLayout eik_layout(double cells) {
     EikLayout l;
+    if (cells <= kEikNarrowCells) l.h = 8, l.tw = 24;
     const char *e = getenv("SSSI_EIK");
     if (!e || !*e) return l;
     if (!strcmp(e, "plain")) {
@@ -444,9 +455,10 @@ static EikLayout eik_layout() {
     if (sscanf(e, "%dx%d", &h, &tw) == 2) {
         l.h = h;
         l.tw = tw;
-        if ((h == 4 && (tw == 32 || tw == 64)) || (h == 8 && (tw == 48 || tw == 64))) return l;
+        if ((h == 4 && (tw == 32 || tw == 64)) || (h == 8 && (tw == 24 || tw == 48 || tw == 64)))
+            return l;
     }
-    fail(SSSI_EINVAL, "SSSI_EIK must be plain, 4x32, 4x64, 8x48 or 8x64 (got \"%s\")", e);
+    fail(SSSI_EINVAL, "SSSI_EIK must be plain, 4x32, 4x64, 8x24, 8x48 or 8x64 (got \"%s\")", e);
 }
 
 // ---------------------------------------------------------------------------
@@ -498,7 +510,7 @@ class Eikonal2D {
         SSSI_HIP(hipEventCreate(&ev[0]));
         SSSI_HIP(hipEventCreate(&ev[1]));
         SSSI_HIP(hipEventRecord(ev[0], stream));
-        const EikLayout lay = eik_layout();
+        const EikLayout lay = eik_layout((double)nn * nsrc);
         if (lay.h == 0) {
             for (int p = 0; p < 4 * iMax; ++p) {
                 hipLaunchKernelGGL(eik_pass, dim3(grid_blocks(total)), dim3(256), 0, stream,
