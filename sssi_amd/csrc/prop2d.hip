@@ -613,14 +613,18 @@ class Prop2D final : public Prop {
     void run_steps(int64_t t_first, int64_t count, bool reverse, bool record,
                    const SnapSink *sink, int K, LaunchStats *st) {
         if (!ap[0].p) {
-            for (auto &b : ap) {
-                b.alloc(g->p[0].n);
-                SSSI_HIP(hipMemsetAsync(b.p, 0, b.bytes(), stream));  // (its padding stays 0)
-            }
+            // held only once all of it is there: the call may fail and come again
+            DevBuf<float> p0(g->p[0].n), p1(g->p[1].n), zpsi, xpsi;
             if (nB > 0) {
-                azpsi.alloc(g->zpsi.n);
-                axpsi.alloc(g->xpsi.n);
+                zpsi.alloc(g->zpsi.n);
+                xpsi.alloc(g->xpsi.n);
             }
+            for (auto *b : {&p0, &p1})  // (their padding stays 0)
+                SSSI_HIP(hipMemsetAsync(b->p, 0, b->bytes(), stream));
+            azpsi = std::move(zpsi);
+            axpsi = std::move(xpsi);
+            ap[0] = std::move(p0);
+            ap[1] = std::move(p1);
         }
         for (int64_t q = 0; q < count;) {
             const int n = (int)std::min<int64_t>(K, count - q);
