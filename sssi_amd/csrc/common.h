@@ -76,11 +76,14 @@ struct DevBuf {
     ~DevBuf() { release(); }
     void alloc(size_t count) {
         release();
-        n = count;
         as = alloc_stream();
-        if (!count) return;
-        if (as) SSSI_HIP(hipMallocAsync((void **)&p, count * sizeof(T), as));
-        else SSSI_HIP(hipMalloc((void **)&p, count * sizeof(T)));
+        if (count) {
+            void *q = nullptr;
+            if (as) SSSI_HIP(hipMallocAsync(&q, count * sizeof(T), as));
+            else SSSI_HIP(hipMalloc(&q, count * sizeof(T)));
+            p = (T *)q;
+        }
+        n = count;  // (0 after a failed allocation: holders compare n)
     }
     void release() {
         if (p) {
@@ -137,8 +140,12 @@ struct HostBuf {
     ~HostBuf() { release(); }
     void alloc(size_t count) {
         release();
-        n = count;
-        if (count) SSSI_HIP(hipHostMalloc((void **)&p, count * sizeof(T), hipHostMallocDefault));
+        if (count) {
+            void *q = nullptr;
+            SSSI_HIP(hipHostMalloc(&q, count * sizeof(T), hipHostMallocDefault));
+            p = (T *)q;
+        }
+        n = count;  // (0 after a failed allocation)
     }
     void release() {
         if (p) (void)hipHostFree(p);
