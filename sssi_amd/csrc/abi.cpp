@@ -80,6 +80,8 @@ PointList dense_to_points(const double *src, int64_t nz, int64_t nx, int64_t ny,
 // layout.  Snapshots go through a device staging buffer of at most ~256 MB.
 void run_oneshot(Prop &P, int64_t nt, bool reverse, double *data, double *snap, int64_t stride) {
     const int64_t cells = P.cells();
+    // (t = 0 alone, whatever lies beyond nt; the kernels' stride is 32 bits wide)
+    stride = std::min(stride, nt);
     const int64_t nsnap = (nt + stride - 1) / stride;
     if (!snap) {
         P.run(reverse ? nt - 1 : 0, nt, reverse, data != nullptr, nullptr, nullptr);

@@ -316,7 +316,7 @@ static void na_run(const double *v, int64_t nz, int64_t nx, int64_t nt, int nsrc
 
     // ---- time loop; with snapshots, segment k runs steps k*stride .. and
     // slice k is written at its first step, then converted and copied out
-    const int64_t stride = snapshot ? snap_stride : nt;
+    const int64_t stride = snapshot ? std::min(snap_stride, nt) : nt;
     for (int64_t t0 = 0, k = 0; t0 < nt; t0 += stride, ++k) {
         const int64_t t1 = std::min(nt, t0 + stride);
         Job2D Jk = J;
