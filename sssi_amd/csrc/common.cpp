@@ -2,6 +2,7 @@
 #include "common.h"
 
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -209,6 +210,45 @@ struct PinnedChunk {
         SSSI_HIP(hipHostMalloc(&p, kChunkBytes, hipHostMallocPortable));
     }
 };
+
+// What stream_to_host's workers share: they sleep on `go` until the next chunk
+// has come (or `stop`), the caller on `through` until a buffer is free again.
+struct Relay {
+    std::mutex mu;
+    std::condition_variable go, through;
+    bool stop = false;
+    size_t ready = 0, team = 0;  // chunks that have come; workers there are
+    std::vector<size_t> done;    // workers that are through with a chunk
+};
+
+// The workers; left early (an exception), they are told to stop and joined.
+struct Crew {
+    Relay &r;
+    std::vector<std::thread> th;
+    template <class F>
+    void start(size_t n, F &f) {
+        try {
+            th.reserve(n);
+            for (size_t k = 0; k < n; ++k) th.emplace_back([&f, k] { f(k); });
+        } catch (const std::system_error &) {  // no more threads: those there do it
+        } catch (const std::bad_alloc &) {
+        }
+        std::lock_guard<std::mutex> lk(r.mu);
+        r.team = th.size();
+    }
+    void join() {
+        for (auto &t : th)
+            if (t.joinable()) t.join();
+    }
+    ~Crew() {
+        {
+            std::lock_guard<std::mutex> lk(r.mu);
+            r.stop = true;
+        }
+        r.go.notify_all();
+        join();
+    }
+};
 }  // namespace
 
 void stream_to_host(const void *dev, size_t n, size_t elem, hipStream_t s, const HostUse &use) {
@@ -223,53 +263,46 @@ void stream_to_host(const void *dev, size_t n, size_t elem, hipStream_t s, const
                                 std::min(per, n - c * per) * elem, hipMemcpyDeviceToHost, s));
         SSSI_HIP(hipStreamSynchronize(s));
     };
+    // what the stream still computes, before any worker waits for it
+    SSSI_HIP(hipStreamSynchronize(s));
     // a worker per MB, up to 15; none for a small result
     const size_t want = std::min<size_t>({15, n * elem >> 20,
                                           std::max(1u, std::thread::hardware_concurrency())});
-    std::vector<std::thread> workers;
-    std::atomic<size_t> ready{0}, team{0};
-    std::atomic<bool> stop{false};
-    std::vector<std::atomic<size_t>> done(nchunk);
-    for (auto &d : done) d.store(0);
+    Relay r;
+    r.done.assign(nchunk, 0);
     auto work = [&](size_t k) {
-        while (team.load(std::memory_order_acquire) == 0) {
-            if (stop.load(std::memory_order_acquire)) return;
-            std::this_thread::yield();
-        }
-        const size_t T = team.load(std::memory_order_acquire);
+        std::unique_lock<std::mutex> lk(r.mu);
         for (size_t c = 0; c < nchunk; ++c) {
-            while (ready.load(std::memory_order_acquire) <= c) {
-                if (stop.load(std::memory_order_acquire)) return;
-                std::this_thread::yield();
-            }
+            r.go.wait(lk, [&] { return r.stop || (r.team > 0 && r.ready > c); });
+            if (r.stop) return;
+            const size_t T = r.team;
+            lk.unlock();
             const size_t m = std::min(per, n - c * per), a = m * k / T, b = m * (k + 1) / T;
             if (b > a) use((const char *)buf[c & 1].p + a * elem, c * per + a, b - a);
-            done[c].fetch_add(1, std::memory_order_release);
+            lk.lock();
+            if (++r.done[c] == T) r.through.notify_one();
         }
     };
-    if (want > 1) {
-        workers.reserve(want);
-        try {
-            for (size_t k = 0; k < want; ++k) workers.emplace_back(work, k);
-        } catch (const std::system_error &) {  // no more threads: those there do it
+    Crew crew{r};  // (last: joined before anything the workers use is gone)
+    if (want > 1) crew.start(want, work);
+    const size_t T = crew.th.size();
+    for (size_t c = 0; c < nchunk; ++c) {
+        if (T > 0 && c >= 2) {  // the buffer's last chunk has been used
+            std::unique_lock<std::mutex> lk(r.mu);
+            r.through.wait(lk, [&] { return r.done[c - 2] == T; });
+        }
+        fetch(c);
+        if (T > 0) {
+            {
+                std::lock_guard<std::mutex> lk(r.mu);
+                r.ready = c + 1;
+            }
+            r.go.notify_all();
+        } else {
+            use(buf[c & 1].p, c * per, std::min(per, n - c * per));
         }
     }
-    const size_t T = workers.size();
-    try {
-        if (T > 0) team.store(T, std::memory_order_release);
-        for (size_t c = 0; c < nchunk; ++c) {
-            if (T > 0 && c >= 2)  // the buffer's last chunk has been used
-                while (done[c - 2].load(std::memory_order_acquire) < T) std::this_thread::yield();
-            fetch(c);
-            if (T > 0) ready.store(c + 1, std::memory_order_release);
-            else use(buf[c & 1].p, c * per, std::min(per, n - c * per));
-        }
-    } catch (...) {
-        stop.store(true, std::memory_order_release);
-        for (auto &t : workers) t.join();
-        throw;
-    }
-    for (auto &t : workers) t.join();
+    crew.join();
 }
 
 void copy_to_host(void *dst, const void *dev, size_t bytes, hipStream_t s) {

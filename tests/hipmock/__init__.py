@@ -13,10 +13,13 @@ LIB = os.path.join(HERE, "_build", "libhipmock.so")
 _HEAD = f"""
 import ctypes
 M = ctypes.CDLL({LIB!r}, mode=ctypes.RTLD_GLOBAL)
-for f in ("hipmock_mallocs", "hipmock_host_mallocs", "hipmock_count", "hipmock_arg"):
+for f in ("hipmock_mallocs", "hipmock_host_mallocs", "hipmock_count", "hipmock_arg",
+          "hipmock_new_left"):
     getattr(M, f).restype = ctypes.c_long
-for f in ("hipmock_fail_malloc", "hipmock_sync_us", "hipmock_copy_limit"):
+for f in ("hipmock_fail_malloc", "hipmock_sync_us", "hipmock_copy_limit",
+          "hipmock_fail_new"):
     getattr(M, f).argtypes = [ctypes.c_long]
+M.hipmock_size.restype = ctypes.c_size_t
 M.hipmock_mem_free.argtypes = [ctypes.c_size_t]
 def watch(name, *sizes):
     M.hipmock_watch(name.encode(), (ctypes.c_size_t * len(sizes))(*sizes), len(sizes))

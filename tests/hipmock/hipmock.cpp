@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <unistd.h>
 
+#include <new>
+
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
@@ -17,6 +19,7 @@
 namespace {
 std::mutex mu;
 std::map<const void *, std::string> kernels;
+std::map<const void *, size_t> sizes;  // device allocations
 struct Launch {
     std::string name;
     unsigned grid[3], block[3];
@@ -32,11 +35,22 @@ std::atomic<size_t> mem_free{(size_t)1 << 38};
 dim3 cfg_grid, cfg_block;
 int dummy;
 
+thread_local long new_in = -1;  // this thread's operator new calls until one throws
+
 hipError_t take(void **p, size_t n) {
     ++n_malloc;
     if (fail_in >= 0 && fail_in-- == 0) return hipErrorOutOfMemory;
     *p = std::calloc(n ? n : 1, 1);
+    std::lock_guard<std::mutex> lk(mu);
+    sizes[*p] = n;
     return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+void drop(void *p) {
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        sizes.erase(p);
+    }
+    std::free(p);
 }
 hipError_t copy(void *d, const void *s, size_t n) {
     n_copied += (long)n;
@@ -45,12 +59,27 @@ hipError_t copy(void *d, const void *s, size_t n) {
 }
 }  // namespace
 
+void *operator new(size_t n) {
+    if (new_in >= 0 && new_in-- == 0) throw std::bad_alloc();
+    if (void *p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+
 extern "C" {
+// the calling thread's k-th operator new from here on throws; what is left of k
+void hipmock_fail_new(long k) { new_in = k; }
+long hipmock_new_left() { return new_in; }
 void hipmock_fail_malloc(long k) { fail_in = k; }
 void hipmock_sync_us(long us) { sync_us = us; }
 void hipmock_copy_limit(long n) { copy_limit = n; }
 void hipmock_mem_free(size_t n) { mem_free = n; }
 long hipmock_mallocs() { return n_malloc; }
+// bytes of the device allocation at p (0: none)
+size_t hipmock_size(const void *p) {
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = sizes.find(p);
+    return it == sizes.end() ? 0 : it->second;
+}
 long hipmock_host_mallocs() { return n_host; }
 void hipmock_watch(const char *name, const size_t *bytes, int n) {
     watch = name;
@@ -117,8 +146,8 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, h
 }
 hipError_t hipMalloc(void **p, size_t n) { return take(p, n); }
 hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return take(p, n); }
-hipError_t hipFree(void *p) { std::free(p); return hipSuccess; }
-hipError_t hipFreeAsync(void *p, hipStream_t) { std::free(p); return hipSuccess; }
+hipError_t hipFree(void *p) { drop(p); return hipSuccess; }
+hipError_t hipFreeAsync(void *p, hipStream_t) { drop(p); return hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     ++n_host;
     *p = std::calloc(n ? n : 1, 1);
