@@ -97,3 +97,29 @@ print("ok")
 
 def test_failed_host_allocation_is_an_error_code():
     assert "ok" in hipmock.run(_NEW_FAILS)
+
+
+_POOL = """
+import threading
+Ps = []
+for _ in range(8):
+    P = sssi_amd.Propagator(np.full((8, 3000), 2000.0, order="F"), 1, 0, 10.0, 10.0, 1e-3)
+    P.set_points([0], [1], np.zeros(1000))
+    P.run(1000)
+    Ps.append(P)
+M.hipmock_sync_us(20000)  # every call holds its chunks while the others start
+def once():
+    th = [threading.Thread(target=P.data, args=(1000,)) for P in Ps]
+    for t in th: t.start()
+    for t in th: t.join()
+once()
+n = M.hipmock_host_mallocs()
+for _ in range(3): once()
+print(M.hipmock_host_mallocs() - n)
+"""
+
+
+def test_concurrent_calls_find_their_chunks():
+    """Eight callers at a time: after the first round no pinned memory is
+    allocated."""
+    assert int(hipmock.run(_POOL)) == 0
