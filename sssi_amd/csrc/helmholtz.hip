@@ -28,8 +28,11 @@
 //   freq_subst   one workgroup per right-hand side, a panel at a time: forward
 //                sweep with the interchanges, column-oriented backward sweep,
 //                the band window of the right-hand side in LDS.
-// Bands too wide for rows in registers (kl > kMaxBand) take freq_panel and
-// freq_trail (global memory) and freq_solve (one step at a time).
+// Bands too wide for rows in registers (kl > kMaxBand) take the column replay:
+//   freq_panel   one workgroup factors the panel, in LDS where its rows fit;
+//   freq_trail(_lds)  workgroups of one to four later columns within reach
+//                replay the panel's interchanges and updates in pivot order;
+//   freq_solve   one workgroup per right-hand side, one step at a time.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -134,28 +137,59 @@ struct LuState {
     int singular;      // first zero pivot column + 1 (0: none)
 };
 
-// Wide bands: factor panel columns j0 .. j0+kNB-1 in global memory (256
-// threads).  Per column: pivot search (wave reductions), the row swap, then
-// each thread scales its rows of the column and applies them to the later
-// columns (the multiplier stays in a register: one pass, no barrier between
-// the two).
+// Column-replay form: factor panel columns j0 .. j0+kNB-1 (256 threads).  With LDS, the panel's
+// rows j0 .. j0+kNB-1+kl (R of them) are staged in dynamic LDS, column-major,
+// for the whole factorisation; entries outside the band are neither read nor
+// written (none of the steps touches them).  Per column: pivot search (wave
+// reductions), the decision by thread 0, the row swap, then each thread
+// scales its rows of the column and applies them to the later columns (the
+// multiplier stays in a register: one pass, no barrier between the two).
+// Measured per panel of 16 columns at kl = 360: 62.7 us with 256 threads,
+// 75.7 us with 1024 (rank-1 split over column groups), 75.1 us with the rows
+// batched through registers.
+template <bool LDS>
 __global__ void __launch_bounds__(256) freq_panel(BandDesc B, int64_t j0, int64_t *__restrict__ piv,
-                                                  int64_t *__restrict__ juv, LuState *st) {
+                                                  int64_t *__restrict__ juv, LuState *st,
+                                                  int64_t R) {
 #pragma clang fp contract(off)
+    extern __shared__ cx P[];
     __shared__ double s_best[4];
     __shared__ int s_arg[4];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int64_t n = B.n, kl = B.kl, ku = B.ku;
     const int64_t jend = min(j0 + kNB, n);
+    const int Ri = (int)R;
+    auto inband = [&](int64_t i, int64_t j) {
+        return i < n && j < n && i - j <= kl && j - i <= kl + ku;
+    };
+    auto A = [&](int64_t i, int64_t j) -> cx & {
+        if constexpr (LDS) return P[(int)(j - j0) * Ri + (int)(i - j0)];
+        else return B.at(i, j);
+    };
+    if constexpr (LDS) {
+        // a row's kNB entries are loaded together, then stored to LDS: one
+        // memory latency per row instead of one per entry
+        for (int r = tid; r < Ri; r += 256) {
+            cx v[kNB];
+#pragma unroll
+            for (int c = 0; c < kNB; ++c) {
+                const int64_t i = j0 + r, j = j0 + c;
+                v[c] = inband(i, j) ? B.at(i, j) : cx{0.0, 0.0};
+            }
+#pragma unroll
+            for (int c = 0; c < kNB; ++c) P[c * Ri + r] = v[c];
+        }
+    }
     // furthest column any step so far reaches (kept by every thread alike)
     int64_t ju = st->ju;
+    __syncthreads();
     for (int64_t j = j0; j < jend; ++j) {
         const int km = (int)min(kl, n - 1 - j);
         // pivot: first maximum of |re| + |im| over rows j .. j+km
         double best = -1.0;
         int arg = 0;
         for (int t = tid; t <= km; t += 256) {
-            const cx a = B.at(j + t, j);
+            const cx a = A(j + t, j);
             const double s = fabs(a.re) + fabs(a.im);
             if (s > best) { best = s; arg = t; }
         }
@@ -183,21 +217,45 @@ __global__ void __launch_bounds__(256) freq_panel(BandDesc B, int64_t j0, int64_
         const int64_t cend = min(jend - 1, ju);  // panel columns within reach
         if (jp != 0 && j + tid <= cend) {
             const int64_t c = j + tid;
-            const cx t = B.at(j, c);
-            B.at(j, c) = B.at(j + jp, c);
-            B.at(j + jp, c) = t;
+            const cx t = A(j, c);
+            A(j, c) = A(j + jp, c);
+            A(j + jp, c) = t;
         }
         __syncthreads();
         if (km > 0) {
-            const cx r = crecip(B.at(j, j));
+            const cx r = crecip(A(j, j));
             for (int t = 1 + tid; t <= km; t += 256) {
-                const cx l = cmul(B.at(j + t, j), r);
-                B.at(j + t, j) = l;
-                for (int64_t c = j + 1; c <= cend; ++c)
-                    B.at(j + t, c) = csub_mul(B.at(j + t, c), l, B.at(j, c));
+                const cx l = cmul(A(j + t, j), r);
+                A(j + t, j) = l;
+                // columns four at a time: their loads are independent and go
+                // out together (each entry's update is the same operation)
+                int64_t c = j + 1;
+                for (; c + 3 <= cend; c += 4) {
+                    cx a[4], u[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        a[q] = A(j + t, c + q);
+                        u[q] = A(j, c + q);
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) A(j + t, c + q) = csub_mul(a[q], l, u[q]);
+                }
+                for (; c <= cend; ++c) A(j + t, c) = csub_mul(A(j + t, c), l, A(j, c));
             }
         }
         __syncthreads();
+    }
+    if constexpr (LDS) {
+        for (int r = tid; r < Ri; r += 256) {
+            cx v[kNB];
+#pragma unroll
+            for (int c = 0; c < kNB; ++c) v[c] = P[c * Ri + r];
+#pragma unroll
+            for (int c = 0; c < kNB; ++c) {
+                const int64_t i = j0 + r, j = j0 + c;
+                if (inband(i, j)) B.at(i, j) = v[c];
+            }
+        }
     }
     if (tid == 0) st->ju = ju;
 }
@@ -230,6 +288,97 @@ __global__ void __launch_bounds__(256) freq_trail(BandDesc B, int64_t j0,
     }
 }
 
+// The same with the column's rows j0 .. j0+R-1 staged in LDS, and all of a
+// thread's multipliers of the panel (rows tid + 256 q, q < RPT), the panel's
+// pivots and reaches loaded up front, so the 16 steps touch only LDS and
+// registers.
+template <int RPT, int NC>
+__global__ void __launch_bounds__(256) freq_trail_lds(BandDesc B, int64_t j0,
+                                                      const int64_t *__restrict__ piv,
+                                                      const int64_t *__restrict__ juv, int64_t R) {
+#pragma clang fp contract(off)
+    __shared__ cx Cl[NC][RPT * 256];
+    __shared__ int64_t s_jv[kNB], s_pv[kNB];
+    const int64_t n = B.n, kl = B.kl, ku = B.ku;
+    const int64_t c0 = j0 + kNB + (int64_t)blockIdx.x * NC;  // columns c0 .. c0+NC-1
+    const int64_t jend = min(j0 + kNB, n);
+    const int tid = threadIdx.x;
+    auto inband = [&](int64_t i, int64_t c) {
+        return c < n && i < n && i - c <= kl && c - i <= kl + ku;
+    };
+    // The reaches, pivots and the columns' rows go out together; the panel's
+    // multipliers are loaded one step ahead of their use (two register sets)
+    // and serve all NC columns of the workgroup.
+    const int64_t reach = juv[jend - 1];
+    if (tid < kNB) {
+        s_jv[tid] = j0 + tid < jend ? juv[j0 + tid] : -1;
+        s_pv[tid] = j0 + tid < jend ? piv[j0 + tid] : j0 + tid;
+    }
+    cx col[NC][RPT];
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const int64_t r = tid + 256 * q;
+            col[k][q] = r < R && inband(j0 + r, c0 + k) ? B.at(j0 + r, c0 + k) : cx{0.0, 0.0};
+        }
+    // multiplier of local row r at step p: L(j0 + r, p) when p < j0 + r <= p + km(p)
+    auto lmul = [&](int pp, cx (&L)[RPT]) {
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const int64_t p = j0 + pp, i = j0 + tid + 256 * q;
+            L[q] = (pp < kNB && p < jend && i > p && i <= p + min(kl, n - 1 - p)) ? B.at(i, p)
+                                                                                : cx{0.0, 0.0};
+        }
+    };
+    cx La[RPT], Lb[RPT];
+    lmul(0, La);
+    if (c0 >= n || c0 > reach) return;  // every column beyond every step's reach: untouched
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const int64_t r = tid + 256 * q;
+            if (r < R) Cl[k][r] = col[k][q];
+        }
+    __syncthreads();
+    auto step = [&](int pp, const cx (&L)[RPT], cx (&Ln)[RPT]) {
+        lmul(pp + 1, Ln);
+        const int64_t p = j0 + pp, jv = s_jv[pp];
+        if (c0 > jv) return;  // block-uniform: no column of the block within reach
+        const int64_t jp = s_pv[pp] - p;
+        // column k within reach (block-uniform; the columns within reach are a prefix)
+        if (jp != 0 && tid < NC && c0 + tid <= jv && c0 + tid < n) {
+            cx *C = Cl[tid];
+            const cx t = C[pp];
+            C[pp] = C[pp + jp];
+            C[pp + jp] = t;
+        }
+        __syncthreads();
+        const int64_t km = min(kl, n - 1 - p);
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            if (c0 + k > jv) break;
+            const cx u = Cl[k][pp];
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+                const int64_t r = tid + 256 * q, i = j0 + r;
+                if (i > p && i <= p + km) Cl[k][r] = csub_mul(Cl[k][r], L[q], u);
+            }
+        }
+        __syncthreads();
+    };
+#pragma unroll 1
+    for (int pp = 0; pp < kNB; pp += 2) {
+        step(pp, La, Lb);
+        step(pp + 1, Lb, La);
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+        for (int64_t r = tid; r < R; r += 256)
+            if (inband(j0 + r, c0 + k)) B.at(j0 + r, c0 + k) = Cl[k][r];
+}
+
 // ---------------------------------------------------------------------------
 // Blocked form, rows in registers.
 //
@@ -243,7 +392,7 @@ __global__ void __launch_bounds__(256) freq_trail(BandDesc B, int64_t j0,
 // through kNB independent updates, and each is stored at its pos -- the
 // operations of the interleaved interchanges and updates, in the same order
 // for each element, with no barrier between the steps.
-constexpr int kMaxRows = 1024;               // rows of a panel and the one before it
+constexpr int kMaxRows = 512;                 // rows of a panel and the one before it
 constexpr int kMaxBand = kMaxRows - 2 * kNB;  // widest kl of the blocked form
 constexpr int kTrailCols = 4;                // columns per workgroup behind the next panel
 
@@ -590,9 +739,9 @@ __device__ __forceinline__ bool quot_ok(double a, double b) {
 // rows jb-kl-ku .. jb+kNB-1), the windows a power-of-two ring in LDS (slot of
 // b[i] = i & mask).  Per panel the first wavefront runs the kNB dependent
 // steps on kNB lanes (values passed by DPP), then every thread applies them to
-// its rows (QF, QB per thread); a panel's factors are loaded into registers
+// its rows (one and QB per thread); a panel's factors are loaded into registers
 // while the dependent steps before them run.
-template <int QF, int QB>
+template <int QB>
 __global__ void __launch_bounds__(512) freq_subst(BandDesc B, LuPanels W, const cx *__restrict__ S,
                                                   cx *__restrict__ U, int64_t mask) {
 #pragma clang fp contract(off)
@@ -611,17 +760,14 @@ __global__ void __launch_bounds__(512) freq_subst(BandDesc B, LuPanels W, const 
 
     // ---- forward
     for (int64_t i = tid; i < min<int64_t>(R, n); i += T) ring[i & mask] = cx{-s[i].re, -s[i].im};
-    cx l[QF][kNB];
-    int ps[QF];
-    auto load_f = [&](int64_t q) {  // the rows' multipliers and positions
+    cx l[kNB];
+    int ps = 0;
+    auto load_f = [&](int64_t q) {  // the row's multipliers and position
         if (q >= np) return;
+        const int r = min(tid, R - 1);
+        ps = W.pos[q * R + r];
 #pragma unroll
-        for (int m = 0; m < QF; ++m) {
-            const int r = min(tid + T * m, R - 1);
-            ps[m] = W.pos[q * R + r];
-#pragma unroll
-            for (int p = 0; p < kNB; ++p) l[m][p] = at(W.L + (q * kNB + p) * R, r);
-        }
+        for (int p = 0; p < kNB; ++p) l[p] = at(W.L + (q * kNB + p) * R, r);
     };
     load_f(0);
     __syncthreads();
@@ -632,17 +778,12 @@ __global__ void __launch_bounds__(512) freq_subst(BandDesc B, LuPanels W, const 
         const int64_t e = j0 + R + tid;
         cx in{0.0, 0.0};
         if (tid < kNB && e < n) in = cx{-s[e].re, -s[e].im};
-        cx x[QF];
+        // (rows past the last are 0: a 0 multiplier must not meet a NaN)
+        cx x = tid < R && j0 + tid < n ? ring[(j0 + tid) & mask] : cx{0.0, 0.0};
+        if (tid < R && ps < kNB) {  // the top rows, in their final order
+            xt[ps] = x;
 #pragma unroll
-        for (int m = 0; m < QF; ++m) {
-            // (rows past the last are 0: a 0 multiplier must not meet a NaN)
-            const int r = tid + T * m;
-            x[m] = r < R && j0 + r < n ? ring[(j0 + r) & mask] : cx{0.0, 0.0};
-            if (r < R && ps[m] < kNB) {  // the top rows, in their final order
-                xt[ps[m]] = x[m];
-#pragma unroll
-                for (int p = 0; p < kNB; ++p) tri[0][p][ps[m]] = l[m][p];
-            }
+            for (int p = 0; p < kNB; ++p) tri[0][p][ps] = l[p];
         }
         __syncthreads();  // the ring has been read
         if (first) {
@@ -657,14 +798,8 @@ __global__ void __launch_bounds__(512) freq_subst(BandDesc B, LuPanels W, const 
         }
         __syncthreads();
 #pragma unroll
-        for (int p = 0; p < kNB; ++p) {
-            const cx up = us[buf][p];
-#pragma unroll
-            for (int m = 0; m < QF; ++m) x[m] = csub_mul(x[m], l[m][p], up);
-        }
-#pragma unroll
-        for (int m = 0; m < QF; ++m)
-            if (tid + T * m < R && ps[m] >= kNB) ring[(j0 + ps[m]) & mask] = x[m];
+        for (int p = 0; p < kNB; ++p) x = csub_mul(x, l[p], us[buf][p]);
+        if (tid < R && ps >= kNB) ring[(j0 + ps) & mask] = x;
         if (tid < kNB && e < n) ring[e & mask] = in;
         __builtin_amdgcn_sched_barrier(0);  // the next panel's loads reuse l's registers
         load_f(q + 1);
@@ -693,14 +828,13 @@ __global__ void __launch_bounds__(512) freq_subst(BandDesc B, LuPanels W, const 
         const int lo = (int)max<int64_t>(p, H - jb);
         return band(jb, e >= lo && e < H && jb + p < n ? (uint32_t)e * (uint32_t)sizeof(cx) : kOut, p);
     };
-    // loaded one block ahead: the rows' entries of the block's columns (of up
-    // to two rows per thread), the pivots (lane p: column p's)
-    constexpr int QP = QB < 2 ? QB : 2;
-    cx w[QP][kNB], piv{1.0, 0.0};
+    // loaded one block ahead: the rows' entries of the block's columns, the
+    // pivots (lane p: column p's)
+    cx w[QB][kNB], piv{1.0, 0.0};
     auto load_b = [&](int64_t jb) {
         if (jb < 0) return;
 #pragma unroll
-        for (int m = 0; m < QP; ++m)
+        for (int m = 0; m < QB; ++m)
 #pragma unroll
             for (int p = 0; p < kNB; ++p) w[m][p] = entry(jb, tid + T * m, p);
         if (tid < kNB) piv = jb + tid < n ? at(B.ab + (jb + tid) * B.ldab, H) : cx{1.0, 0.0};
@@ -754,7 +888,7 @@ __global__ void __launch_bounds__(512) freq_subst(BandDesc B, LuPanels W, const 
             cx x = live ? ring[i & mask] : cx{0.0, 0.0};
 #pragma unroll
             for (int p = kNB - 1; p >= 0; --p)
-                x = csub_mul(x, m < QP ? w[m < QP ? m : 0][p] : entry(jb, r, p), us[buf][p]);
+                x = csub_mul(x, w[m][p], us[buf][p]);
             if (live) ring[i & mask] = x;
             __builtin_amdgcn_sched_barrier(0);  // (the next block's loads reuse w's registers)
         }
@@ -766,7 +900,7 @@ __global__ void __launch_bounds__(512) freq_subst(BandDesc B, LuPanels W, const 
     }
 }
 
-// Wide bands: one right-hand side per workgroup of 1024: b = -s, forward sweep with
+// Column-replay form: one right-hand side per workgroup of 1024: b = -s, forward sweep with
 // interchanges (window b[j .. j+kl]), backward sweep (window b[j-kl-ku .. j]),
 // the windows a power-of-two ring in LDS (slot of b[q] = q & mask).  The
 // values entering the window come from global memory in chunks of 1024 per
@@ -966,14 +1100,28 @@ static void freq_validate(const double *m, int64_t nz, int64_t nx, double w, int
 struct FreqSystem {
     int64_t nz, nx, n, kl, ku, ldab;
     int k;
+    bool form_blocked;
     OwnedStream s;  // before the buffers: destroyed after them
     DevBuf<cx> ab;
-    DevBuf<int64_t> piv, juv;  // wide bands: per column
+    DevBuf<int64_t> piv, juv;  // column-replay form: per column
     DevBuf<cx> lp;             // blocked form (LuPanels)
     DevBuf<int> pos;
     DevBuf<int64_t> reach;
     DevBuf<LuState> st;
-    bool blocked() const { return kl <= kMaxBand; }
+    // Blocked form up to kMaxBand, where a panel's rows still fit 512 threads
+    // with all 16 columns in registers; the column replay beyond (1024 threads
+    // have half the registers each: 145 spilled in the pivot chain).  Whole call
+    // with 20 sources, ms, blocked / replay: band 246 13.7 / 21.5, 360 20.8 /
+    // 36.8, 480 30.4 / 50.3; with 1024 threads 483 86.6 / 50.8, 600 120 / 86, 771
+    // 161 / 154, 900 191 / 187.
+    // SSSI_FREQ_NC = 1, 2 or 4: the column replay at every band, with that many
+    // columns per workgroup.
+    static int replay_columns() {
+        const char *e = std::getenv("SSSI_FREQ_NC");
+        const int v = e ? std::atoi(e) : 0;
+        return v == 1 || v == 2 || v == 4 ? v : 0;
+    }
+    bool blocked() const { return form_blocked; }
     LuPanels panels() const { return LuPanels{lp.p, pos.p, reach.p, (int)(kNB + kl)}; }
 
     FreqSystem(const double *m, int64_t nz_, int64_t nx_, double w, int N, int nB, double dz,
@@ -982,6 +1130,7 @@ struct FreqSystem {
         kl = (int64_t)k * nz;
         ku = kl;
         ldab = 2 * kl + ku + 1;
+        form_blocked = kl <= kMaxBand && replay_columns() == 0;
         if (band && (double)ldab * n * sizeof(cx) > 200e9)
             fail(SSSI_ENOMEM, "band storage of %.1f GB exceeds the device budget",
                  (double)ldab * n * sizeof(cx) / 1e9);
@@ -1053,20 +1202,43 @@ struct FreqSystem {
             const int64_t c0 = (q + 1) * kNB, c1 = std::min(n - 1, q * kNB - 1 + kl + ku);
             const int64_t nt = q > 0 && c1 >= c0 ? (c1 - c0 + kTrailCols) / kTrailCols : 0;
             const dim3 g((unsigned)(1 + nt));
-            const int64_t rows = kl + 2 * kNB;
-            if (rows <= 256)
+            if (kl + 2 * kNB <= 256)
                 hipLaunchKernelGGL(freq_lu<4>, g, dim3(256), 0, s, B, panels(), q, st.p);
-            else if (rows <= 512)
-                hipLaunchKernelGGL(freq_lu<8>, g, dim3(512), 0, s, B, panels(), q, st.p);
             else
-                hipLaunchKernelGGL(freq_lu<16>, g, dim3(1024), 0, s, B, panels(), q, st.p);
+                hipLaunchKernelGGL(freq_lu<8>, g, dim3(512), 0, s, B, panels(), q, st.p);
         }
+        const int64_t R = std::min<int64_t>(n, kNB + kl);  // panel rows (and a column's)
+        const size_t plds = (size_t)kNB * R * sizeof(cx);
+        const bool panel_lds = plds + 1024 <= lds_limit();
+        const int rpt = R <= 256 ? 1 : R <= 512 ? 2 : R <= 1024 ? 4 : 0;
+        // columns per workgroup of the replay: two share one load of the
+        // panel's multipliers (every workgroup reads the same panel, so fewer
+        // workgroups contend less for its cache lines): 1050 replays at kl = 360
+        // take 67.2 ms at 2 columns, 77.3 ms at 1 and 78.5 ms at 4.
+        const int trail_nc = replay_columns() ? replay_columns() : 2;
         for (int64_t j0 = 0; !blocked() && j0 < n; j0 += kNB) {
-            hipLaunchKernelGGL(freq_panel, dim3(1), dim3(256), 0, s, B, j0, piv.p, juv.p, st.p);
+            if (panel_lds)
+                hipLaunchKernelGGL(freq_panel<true>, dim3(1), dim3(256), plds, s, B, j0, piv.p,
+                                   juv.p, st.p, R);
+            else
+                hipLaunchKernelGGL(freq_panel<false>, dim3(1), dim3(256), 0, s, B, j0, piv.p,
+                                   juv.p, st.p, R);
             const int64_t c0 = j0 + kNB, c1 = std::min(n - 1, j0 + kNB - 1 + kl + ku);
             if (c1 < c0) continue;
-            hipLaunchKernelGGL(freq_trail, dim3((unsigned)(c1 - c0 + 1)), dim3(256), 0, s, B, j0,
-                               piv.p, juv.p);
+            const dim3 g((unsigned)(c1 - c0 + 1));
+            const dim3 g2((unsigned)((c1 - c0 + 2) / 2)), g4((unsigned)((c1 - c0 + 4) / 4));
+            switch (rpt * (trail_nc == 4 ? 100 : trail_nc == 2 ? 10 : 1)) {
+                case 1: hipLaunchKernelGGL((freq_trail_lds<1, 1>), g, dim3(256), 0, s, B, j0, piv.p, juv.p, R); break;
+                case 2: hipLaunchKernelGGL((freq_trail_lds<2, 1>), g, dim3(256), 0, s, B, j0, piv.p, juv.p, R); break;
+                case 4: hipLaunchKernelGGL((freq_trail_lds<4, 1>), g, dim3(256), 0, s, B, j0, piv.p, juv.p, R); break;
+                case 10: hipLaunchKernelGGL((freq_trail_lds<1, 2>), g2, dim3(256), 0, s, B, j0, piv.p, juv.p, R); break;
+                case 20: hipLaunchKernelGGL((freq_trail_lds<2, 2>), g2, dim3(256), 0, s, B, j0, piv.p, juv.p, R); break;
+                case 40: hipLaunchKernelGGL((freq_trail_lds<4, 2>), g2, dim3(256), 0, s, B, j0, piv.p, juv.p, R); break;
+                case 100: hipLaunchKernelGGL((freq_trail_lds<1, 4>), g4, dim3(256), 0, s, B, j0, piv.p, juv.p, R); break;
+                case 200: hipLaunchKernelGGL((freq_trail_lds<2, 4>), g4, dim3(256), 0, s, B, j0, piv.p, juv.p, R); break;
+                case 400: hipLaunchKernelGGL((freq_trail_lds<4, 4>), g4, dim3(256), 0, s, B, j0, piv.p, juv.p, R); break;
+                default: hipLaunchKernelGGL(freq_trail, g, dim3(256), 0, s, B, j0, piv.p, juv.p);
+            }
         }
         SSSI_HIP(hipGetLastError());
         SSSI_HIP(hipEventRecord(e1, s));
@@ -1093,7 +1265,7 @@ struct FreqSystem {
                  "nz = %lld; the window of 2 kl + 1 values, rounded up to a power of two, and "
                  "the staging must fit %zu bytes of LDS)", (long long)kl, lds_limit());
         const int64_t rows = kl + ku;  // per step, the backward sweep's is the wider
-        const int rpt = rows <= 2048 ? 2 : rows <= 4096 ? 4 : 8;  // wide bands
+        const int rpt = rows <= 1024 ? 1 : rows <= 2048 ? 2 : rows <= 4096 ? 4 : 8;
         DevBuf<cx> dS((size_t)n * nsrc), dU((size_t)n * nsrc);
         SSSI_HIP(hipMemcpyAsync(dS.p, S, dS.bytes(), hipMemcpyHostToDevice, s));
         BandDesc B{ab.p, n, kl, ku, ldab};
@@ -1104,19 +1276,17 @@ struct FreqSystem {
         const dim3 g((unsigned)nsrc), blk(1024);
         const int64_t mask = ring - 1;
         if (blocked()) {
-            // a thread per row of the backward window up to 512 rows, 2 to 4
-            // rows per thread beyond (kl <= kMaxBand: at most 1984 rows)
+            // a thread per row of the backward window up to 512 rows, two rows
+            // per thread beyond (kl <= kMaxBand: at most 960 rows)
             const dim3 bl((unsigned)std::max<int64_t>(kNB * kNB,
                                                       std::min<int64_t>(512, round_up(rows, 64))));
-#define SSSI_SUBST(QF, QB) \
-    hipLaunchKernelGGL((freq_subst<QF, QB>), g, bl, sh, s, B, panels(), dS.p, dU.p, mask)
-            if (rows <= 512) SSSI_SUBST(1, 1);
-            else if (kNB + kl <= 512) SSSI_SUBST(1, 2);
-            else if (rows <= 1024) SSSI_SUBST(2, 2);
-            else SSSI_SUBST(2, 4);
-#undef SSSI_SUBST
+            if (rows <= 512)
+                hipLaunchKernelGGL(freq_subst<1>, g, bl, sh, s, B, panels(), dS.p, dU.p, mask);
+            else
+                hipLaunchKernelGGL(freq_subst<2>, g, bl, sh, s, B, panels(), dS.p, dU.p, mask);
         } else
             switch (rpt) {
+                case 1: hipLaunchKernelGGL(freq_solve<1>, g, blk, sh, s, B, piv.p, dS.p, dU.p, mask); break;
                 case 2: hipLaunchKernelGGL(freq_solve<2>, g, blk, sh, s, B, piv.p, dS.p, dU.p, mask); break;
                 case 4: hipLaunchKernelGGL(freq_solve<4>, g, blk, sh, s, B, piv.p, dS.p, dU.p, mask); break;
                 default: hipLaunchKernelGGL(freq_solve<8>, g, blk, sh, s, B, piv.p, dS.p, dU.p, mask);

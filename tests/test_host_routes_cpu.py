@@ -1,0 +1,44 @@
+"""Which kernels a call launches, without a GPU: the choice between two forms
+of a kernel where the wrong one gives the same values more slowly."""
+import pytest
+
+import hipmock
+
+_HELM = """
+from sssi_amd import helmholtz
+m = np.full(({nz}, {nx}), 2000.0 ** -2, order="F")
+S = np.zeros(({nz} * {nx}, 1), dtype=np.complex128)
+helmholtz.solve(m, S, 60.0, {N}, 1, 10.0, 10.0)
+for k in ("freq_lu", "freq_subst", "freq_panel", "freq_trail_lds", "freq_trail", "freq_solve"):
+    print(k, count(k))
+"""
+
+
+def _helm(nz, nx, N, **env):
+    out = hipmock.run(_HELM.format(nz=nz, nx=nx, N=N), **env)
+    n = {k: int(v) for k, v in (line.split() for line in out.splitlines())}
+    n["freq_trail"] -= n["freq_trail_lds"]  # (counted by part of the name)
+    return {k for k, v in n.items() if v}
+
+
+BLOCKED = {"freq_lu", "freq_subst"}
+REPLAY = {"freq_panel", "freq_trail_lds", "freq_solve"}
+GLOBAL = {"freq_panel", "freq_trail", "freq_solve"}
+
+
+@pytest.mark.parametrize("nz, nx, N, form", [
+    (40, 10, 1, BLOCKED), (160, 4, 2, BLOCKED),                # bands 40, 480
+    (161, 4, 2, REPLAY), (300, 4, 2, REPLAY),                  # 483, 900
+    (332, 4, 2, REPLAY), (336, 4, 2, REPLAY),                  # 996, 1008: 1024 rows
+    (337, 4, 2, GLOBAL),                                       # 1011
+    (200, 5, 3, REPLAY), (128, 8, 5, REPLAY),                  # 1000, 1152 in 1000, 1024 unknowns
+])
+def test_helmholtz_form(nz, nx, N, form):
+    """Rows of a panel in 512 threads' registers, else in 1024 LDS rows, else
+    in global memory."""
+    assert _helm(nz, nx, N) == form
+
+
+@pytest.mark.parametrize("nc", ["1", "2", "4"])
+def test_helmholtz_replay_on_request(nc):
+    assert _helm(40, 10, 1, SSSI_FREQ_NC=nc) == REPLAY
