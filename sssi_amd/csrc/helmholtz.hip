@@ -1100,7 +1100,7 @@ static void freq_validate(const double *m, int64_t nz, int64_t nx, double w, int
 struct FreqSystem {
     int64_t nz, nx, n, kl, ku, ldab;
     int k;
-    bool form_blocked;
+    bool form_blocked = false;  // (chosen by factor)
     OwnedStream s;  // before the buffers: destroyed after them
     DevBuf<cx> ab;
     DevBuf<int64_t> piv, juv;  // column-replay form: per column
@@ -1122,6 +1122,17 @@ struct FreqSystem {
         return v == 1 || v == 2 || v == 4 ? v : 0;
     }
     bool blocked() const { return form_blocked; }
+    // Whether the panels of the blocked form (a third of the band's bytes on wide
+    // bands, more than its bytes on narrow ones) fit beside what the replay needs
+    // too; looked up where they are large enough to matter.
+    bool panels_fit(int nsrc) const {
+        const int64_t np = (n + kNB - 1) / kNB;
+        const double need = (double)np * (kNB + kl) * (kNB * sizeof(cx) + sizeof(int));
+        if (need < 1e9) return true;
+        size_t free_now = 0, total = 0;
+        SSSI_HIP(hipMemGetInfo(&free_now, &total));
+        return need + 2.0 * n * nsrc * sizeof(cx) + 256e6 <= (double)free_now;
+    }
     LuPanels panels() const { return LuPanels{lp.p, pos.p, reach.p, (int)(kNB + kl)}; }
 
     FreqSystem(const double *m, int64_t nz_, int64_t nx_, double w, int N, int nB, double dz,
@@ -1130,7 +1141,6 @@ struct FreqSystem {
         kl = (int64_t)k * nz;
         ku = kl;
         ldab = 2 * kl + ku + 1;
-        form_blocked = kl <= kMaxBand && replay_columns() == 0;
         if (band && (double)ldab * n * sizeof(cx) > 200e9)
             fail(SSSI_ENOMEM, "band storage of %.1f GB exceeds the device budget",
                  (double)ldab * n * sizeof(cx) / 1e9);
@@ -1180,8 +1190,9 @@ struct FreqSystem {
         return prop.sharedMemPerBlock;
     }
 
-    float factor() {
+    float factor(int nsrc) {
         const int64_t np = (n + kNB - 1) / kNB;
+        form_blocked = kl <= kMaxBand && replay_columns() == 0 && panels_fit(nsrc);
         if (blocked()) {
             lp.alloc((size_t)(np * kNB * (kNB + kl)));
             pos.alloc((size_t)(np * (kNB + kl)));
@@ -1351,7 +1362,7 @@ int sssi_freqCpmlFor2dAw(const double *model, int64_t nz, int64_t nx, const doub
             fail(SSSI_EINVAL, "source and snapshot must hold at least one column");
         FreqSystem fs(model, nz, nx, w, nDiffOrder, nBoundary, dz, dx, true, nullptr, nullptr,
                       nullptr);
-        g_factor_ms = fs.factor();
+        g_factor_ms = fs.factor(nsrc);
         g_solve_ms = fs.solve(source, nsrc, snapshot);
     });
 }

@@ -14,8 +14,8 @@ for k in ("freq_lu", "freq_subst", "freq_panel", "freq_trail_lds", "freq_trail",
 """
 
 
-def _helm(nz, nx, N, **env):
-    out = hipmock.run(_HELM.format(nz=nz, nx=nx, N=N), **env)
+def _helm(nz, nx, N, before="", **env):
+    out = hipmock.run(before + _HELM.format(nz=nz, nx=nx, N=N), **env)
     n = {k: int(v) for k, v in (line.split() for line in out.splitlines())}
     n["freq_trail"] -= n["freq_trail_lds"]  # (counted by part of the name)
     return {k for k, v in n.items() if v}
@@ -42,3 +42,11 @@ def test_helmholtz_form(nz, nx, N, form):
 @pytest.mark.parametrize("nc", ["1", "2", "4"])
 def test_helmholtz_replay_on_request(nc):
     assert _helm(40, 10, 1, SSSI_FREQ_NC=nc) == REPLAY
+
+
+@pytest.mark.parametrize("free, form", [(1 << 38, BLOCKED), (1_300_000_000, REPLAY)])
+def test_helmholtz_panels_that_do_not_fit(free, form):
+    """1.1 GB of panels (band 40, 1.2e6 unknowns) with and without the room for
+    them: without, the form that needs none."""
+    n = _helm(40, 30000, 1, before=f"M.hipmock_mem_free({free})\n")
+    assert n == form
