@@ -251,6 +251,101 @@ __global__ void __launch_bounds__(64 * kSpZ / R) sponge2d_steps(Sponge2dArgs a, 
         sponge2d_tile<R, false>(a, tx, ty, edge);
 }
 
+// One time step: for runs cut into pieces of a step or two, where the tiles of
+// sponge2d_steps would compute 2.7 cells for each one they write and share
+// their trip to memory with nobody.  A wavefront owns 64 columns x RZ rows
+// (lane = column); every load is a raw buffer load with the wave-uniform row
+// offset in the scalar offset: the column window p(i0-1 .. i0+RZ) once, the x
+// neighbours as loads shifted by one column, then p_old and v*dt.  The new
+// level goes where p_old was (ocur: each cell's is read by its own lane alone),
+// with the arithmetic of sponge2d_tile cell by cell.  Rows i0-1 .. i0+RZ and
+// columns j-1 .. j+1 of every wavefront with a row inside the model lie in the
+// padded array, whose padding stays zero: lanes outside store nothing.
+// Bound by the launch on small grids, by four arrays' streams on large ones.
+// A step in pieces of one, this kernel / sponge2d_steps, us: 100 x 150 3.6 /
+// 3.9, 515 x 1203 3.7 / 6.0, 1040 x 3080 7.6 / 15.5; in pieces of two 3.2 / 2.5,
+// 3.6 / 4.0, 7.6 / 9.9; of three 3.0 / 2.0, 3.7 / 3.0, 7.6 / 7.2.
+// 1-D over ntx * ntz block tiles, XCD-banded as sponge2d_steps.
+constexpr int kSpRZ = 4;
+template <int RZ>
+__global__ void __launch_bounds__(256) sponge2d_step(Sponge2dArgs a, int ntx) {
+    const int lane = threadIdx.x & 63, w = wave_id();
+    const int nb = (int)gridDim.x, b = (int)blockIdx.x;
+    const int q = nb / 8, rem = nb % 8, x = b % 8;
+    const int tile = x * q + min(x, rem) + b / 8;
+    const int ty = tile / ntx, tx = tile - ty * ntx;
+    const int j = tx * 64 + lane;
+    const int i0 = (ty * 4 + w) * RZ;
+    if (i0 >= a.nz) return;
+    const bool jin = j < a.nx;
+    const uint32_t rowb = (uint32_t)a.pitch * 4u;
+    const uint32_t nbytes = rowb * (uint32_t)a.rows;
+    const __amdgpu_buffer_rsrc_t rP = buf_rsrc(a.pcur, nbytes);
+    const __amdgpu_buffer_rsrc_t rO = buf_rsrc(a.ocur, nbytes);
+    const __amdgpu_buffer_rsrc_t rV = buf_rsrc(a.vdt, nbytes);
+    const uint32_t vcol = (uint32_t)(j + kHX) * 4u;
+    const uint32_t srow = (uint32_t)(i0 + kHZ) * rowb;
+
+    float col[RZ + 2], cl[RZ], cr[RZ], po[RZ], vd[RZ];
+#pragma unroll
+    for (int r = 0; r < RZ + 2; ++r) col[r] = buf_ld(rP, vcol, srow + (r - 1) * rowb);
+#pragma unroll
+    for (int r = 0; r < RZ; ++r) {
+        cl[r] = buf_ld(rP, vcol - 4u, srow + r * rowb);
+        cr[r] = buf_ld(rP, vcol + 4u, srow + r * rowb);
+        po[r] = buf_ld(rO, vcol, srow + r * rowb);
+        vd[r] = buf_ld(rV, vcol, srow + r * rowb);
+    }
+
+    // damping factor: the bottom strip's by row, else the side strips' by column
+    const int nB = a.nB;
+    float gx = 1.f;
+    if (jin && j < nB) gx = a.g[j];
+    else if (jin && j >= a.nx - nB) gx = a.g[a.nx - 1 - j];
+    // source terms, summed per cell in source order, then surface injection
+    const int t = a.t0;
+    float s[RZ];
+#pragma unroll
+    for (int r = 0; r < RZ; ++r) s[r] = 0.f;
+    if (!a.reverse && t < a.src_nt)
+        for (int k = 0; k < a.nsrc; ++k) {
+            const int cell = ld_uniform(a.src_cell + k);
+            const int ci = cell / a.nx, cj = cell - ci * a.nx;
+            if (ci >= i0 && ci < i0 + RZ && cj == j) {
+                const float amp = ld_uniform(a.src_amp + (size_t)t * a.nsrc + k);
+#pragma unroll
+                for (int r = 0; r < RZ; ++r)
+                    if (ci == i0 + r) s[r] += amp;
+            }
+        }
+    if (a.reverse && a.surf && t < a.surf_nt && i0 == 0 && jin) s[0] += a.surf[(size_t)t * a.nx + j];
+    float *snap = a.snap && t % a.snap_stride == 0
+                      ? a.snap + (size_t)(t / a.snap_stride - a.snap_slot0) * a.nz * a.nx
+                      : nullptr;
+
+    float pn0 = 0.f;
+#pragma unroll
+    for (int r = 0; r < RZ; ++r) {
+        const int i = i0 + r;
+        if (i >= a.nz) break;
+        const float gf = i >= a.nz - nB ? ld_uniform(a.g + (a.nz - 1 - i)) : gx;
+        const float v2 = vd[r] * vd[r];
+        const float ax = v2 * a.idx2, az = v2 * a.idz2;
+        const float pc = col[r + 1];
+        float lap = fmaf(ax, (cr[r] - pc) + (cl[r] - pc), az * ((col[r + 2] - pc) + (col[r] - pc)));
+        lap = fmaf(-s[r], v2, lap);
+        float pn = pc + (lap + fmaf(-gf, po[r], pc));
+        pn *= gf;
+        buf_st(pn, rO, jin ? vcol : kOOB, srow + r * rowb);
+        if (r == 0) pn0 = pn;
+        if (jin) {
+            if (a.rec && i == 0) a.rec[(size_t)t * a.nx + j] = pn;
+            if (snap) snap[(size_t)i * a.nx + j] = pn;
+        }
+    }
+    if (a.health && i0 == 0) report_nonfinite(a.health, jin && nonfinite(pn0), a.step);
+}
+
 // One (slice, y) plane's 64 x 64 tile through LDS: rows of x in, columns of z
 // out, both coalesced; 65 floats per LDS row keep the banks apart.
 __global__ void __launch_bounds__(256) z_fastest(const float *__restrict__ in,
@@ -527,8 +622,8 @@ class Prop2D final : public Prop {
         else launch_nonfinite_scan(sp[cur][0].p, sp[cur][0].n, sp_health.p, (int)done, stream);
     }
 
-    // n <= kSpK sponge steps from time index t
-    void steps_sponge(int64_t t, int n, bool reverse, bool record, const SnapSink *sink,
+    // n <= kSpK sponge steps from time index t; the launches it took
+    int steps_sponge(int64_t t, int n, bool reverse, bool record, const SnapSink *sink,
                       int step) {
         Sponge2dArgs a{};
         a.health = sp_health.p;
@@ -563,6 +658,24 @@ class Prop2D final : public Prop {
         }
         const int ntx = (int)((nx + kSpCX - 1) / kSpCX);
         const int64_t ntz = (nz + kSpCZ - 1) / kSpCZ;
+        // single steps: one at a time, and two where the chip is full (the
+        // figures at sponge2d_step)
+        if (n == 1 || (n == 2 && ntx * ntz >= 512)) {
+            const int ntx1 = (int)((nx + 63) / 64);
+            const int64_t ntz1 = (nz + 4 * kSpRZ - 1) / (4 * kSpRZ);
+            for (int q = 0; q < n; ++q) {
+                a.t0 = (int)(reverse ? t - q : t + q);
+                a.step = step + q;
+                a.nsteps = 1;
+                a.pcur = sp[cur][0].p;
+                a.ocur = sp[cur][1].p;  // (in place of the old level)
+                hipLaunchKernelGGL(sponge2d_step<kSpRZ>, dim3((unsigned)(ntx1 * ntz1)), dim3(256),
+                                   0, stream, a, ntx1);
+                SSSI_HIP(hipGetLastError());
+                std::swap(sp[cur][0], sp[cur][1]);
+            }
+            return n;
+        }
         // 4 rows per wave while the tiles (8 waves each) leave the chip's 1024
         // SIMDs idle or nearly so, 8 rows from two blocks per CU
         const dim3 grid((unsigned)(ntx * ntz));
@@ -572,6 +685,7 @@ class Prop2D final : public Prop {
             hipLaunchKernelGGL(sponge2d_steps<8>, grid, dim3(64 * kSpZ / 8), 0, stream, a, ntx);
         SSSI_HIP(hipGetLastError());
         cur ^= 1;
+        return 1;
     }
 
     void run(int64_t t_first, int64_t count, bool reverse, bool record, const SnapSink *sink,
@@ -599,9 +713,9 @@ class Prop2D final : public Prop {
         }
         for (int64_t q = 0; q < count; q += kSpK) {
             const int n = (int)std::min<int64_t>(kSpK, count - q);
-            steps_sponge(reverse ? t_first - q : t_first + q, n, reverse, record, sink,
-                         (int)(done + q));
-            if (st) st->launches++;
+            const int nl = steps_sponge(reverse ? t_first - q : t_first + q, n, reverse, record,
+                                        sink, (int)(done + q));
+            if (st) st->launches += nl;
         }
         done += count;
         steps_done = done;

@@ -50,3 +50,23 @@ def test_helmholtz_panels_that_do_not_fit(free, form):
     them: without, the form that needs none."""
     n = _helm(40, 30000, 1, before=f"M.hipmock_mem_free({free})\n")
     assert n == form
+
+
+_SPONGE = """
+v = np.full(({nz}, {nx}), 2000.0, order="F")
+P = sssi_amd.Propagator(v, 1, 5, 10.0, 10.0, 1e-3, abc="sponge")
+P.set_points([0], [1], np.zeros(64))
+M.hipmock_clear()
+P.run_steps(0, {n})
+print(count("sponge2d_stepILi"), count("sponge2d_steps"))
+"""
+
+
+@pytest.mark.parametrize("nz, nx, n, single, several", [
+    (100, 150, 1, 1, 0), (100, 150, 2, 0, 1), (100, 150, 8, 0, 1), (100, 150, 17, 1, 2),
+    (515, 1203, 1, 1, 0), (515, 1203, 2, 2, 0), (515, 1203, 3, 0, 1), (515, 1203, 10, 2, 1),
+])
+def test_sponge_pieces(nz, nx, n, single, several):
+    """Pieces of one step, and of two on a full chip, take the one-step kernel."""
+    out = hipmock.run(_SPONGE.format(nz=nz, nx=nx, n=n)).split()
+    assert [int(x) for x in out] == [single, several]
