@@ -753,12 +753,15 @@ struct Steps2D {
     static constexpr int L = 2 * N - 1;
     static constexpr int K = N == 1 ? 8 : N == 2 ? 4 : N == 3 ? 3 : 2;
     static constexpr int R = 4, W = N == 3 ? 12 : 8;
+    static constexpr int FEW = N == 2 ? 8 : kFewSources;  // (WaveSources)
     static constexpr int EZ = R * W, H = K * L, CX = kTX - 2 * H, CZ = EZ - 2 * H;
 };
 
-template <int N>
-__global__ void __launch_bounds__(64 * Steps2D<N>::W) cpml2d_steps(Job2D J, Steps2DOut O, int rz,
-                                                                   int ntx, int step0, int n) {
+// MANY: more than FEW sources (for N <= 2 held to the registers that let two
+// workgroups onto a CU: 300 x 500, N=2 at one source 3.9 us per step, 4.9 without).
+template <int N, bool MANY>
+__global__ void __launch_bounds__(64 * Steps2D<N>::W, MANY && N <= 2 ? 4 : 1)
+    cpml2d_steps(Job2D J, Steps2DOut O, int rz, int ntx, int step0, int n) {
     using T = Steps2D<N>;
     constexpr int L = T::L, R = T::R, EZ = T::EZ, H = T::H, PAD = 16;
     // L (s_az: N) rows of zeros above and below the tile, so that a wave's
@@ -835,12 +838,8 @@ __global__ void __launch_bounds__(64 * Steps2D<N>::W) cpml2d_steps(Job2D J, Step
         }
     }
     // sources among the wave's cells
-    bool has_src = false;
-    if (!J.reverse && J.src_ptr)
-        for (int k = 0; k < J.nsrc; ++k) {
-            const int cell = ld_uniform(J.src_cell + k), ci = cell / nx, cj = cell - ci * nx;
-            has_src |= ci >= i0 && ci < i0 + R && cj >= tx * T::CX - H && cj < tx * T::CX - H + kTX;
-        }
+    WaveSources<R, MANY> src{J.src_cell, J.src_amp, J.nsrc, J.src_nt, nx, i0, tx * T::CX - H};
+    const bool has_src = !J.reverse && J.src_ptr && src.find(rel0);
     const bool top = i0 <= 0 && i0 + R > 0;  // the wave holds row 0
     const bool surf_here = top && J.reverse && J.surf;
 
@@ -967,16 +966,7 @@ __global__ void __launch_bounds__(64 * Steps2D<N>::W) cpml2d_steps(Job2D J, Step
                 float sv[R];
 #pragma unroll
                 for (int r = 0; r < R; ++r) sv[r] = 0.f;
-                if (has_src && t < J.src_nt)
-                    for (int k = 0; k < J.nsrc; ++k) {
-                        const int cell = ld_uniform(J.src_cell + k), ci = cell / nx, cj = cell - ci * nx;
-                        const float a = ld_uniform(J.src_amp + (size_t)t * J.nsrc + k);
-                        if (cj == j) {
-#pragma unroll
-                            for (int r = 0; r < R; ++r)
-                                if (ci == i0 + r) sv[r] += a;
-                        }
-                    }
+                if (has_src) src.add(t, j, sv);
                 if (surf_here && t < J.surf_nt && jin) {
                     const size_t o = (size_t)t * nx + j;
                     const float x = J.surf2 ? J.surf[o] - J.surf2[o] : J.surf[o];
@@ -1468,8 +1458,9 @@ void launch_cpml2d_steps(const Cpml2dGrid &g, const Job2D &job, const Steps2DOut
         using T = Steps2D<NN>;                                                                \
         const int ntx = (int)((g.nx + T::CX - 1) / T::CX);                                    \
         const int ntz = (int)((g.nz + T::CZ - 1) / T::CZ);                                    \
-        hipLaunchKernelGGL(cpml2d_steps<NN>, dim3((unsigned)(ntx * ntz)), dim3(64 * T::W), 0, \
-                           s, job, out, g.rz, ntx, step, n);                                  \
+        auto kernel = job.nsrc > T::FEW ? cpml2d_steps<NN, true> : cpml2d_steps<NN, false>; \
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(ntx * ntz)), dim3(64 * T::W), 0, s, job,   \
+                           out, g.rz, ntx, step, n);                                          \
         break;                                                                                \
     }
     switch (g.N) {

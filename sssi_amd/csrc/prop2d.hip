@@ -61,7 +61,7 @@ __device__ __forceinline__ float lane_right(float v) {
 // Up to kSpK steps on the tile (ty, tx): see sponge2d_steps.  INNER: the whole
 // tile lies inside the model and off its top row, and no damping strip touches
 // it (every factor 1).
-template <int R, bool INNER>
+template <int R, bool INNER, bool MANY>
 __device__ __forceinline__ void sponge2d_tile(const Sponge2dArgs &a, int tx, int ty,
                                               float (&edge)[2][kSpZ / R + 2][2][64]) {
     constexpr int K = kSpK;
@@ -113,13 +113,8 @@ __device__ __forceinline__ void sponge2d_tile(const Sponge2dArgs &a, int tx, int
             if (iin(r) && i0 + r >= a.nz - a.nB) gf[r] = ld_uniform(a.g + (a.nz - 1 - i0 - r));
     }
     // sources in this wave's rows and columns
-    bool has_src = false;
-    if (!a.reverse)
-        for (int k = 0; k < a.nsrc; ++k) {
-            const int cell = ld_uniform(a.src_cell + k);
-            const int ci = cell / a.nx, cj = cell - ci * a.nx;
-            has_src |= ci >= i0 && ci < i0 + R && cj >= tx * kSpCX - K && cj < tx * kSpCX - K + 64;
-        }
+    WaveSources<R, MANY> src{a.src_cell, a.src_amp, a.nsrc, a.src_nt, a.nx, i0, tx * kSpCX - K};
+    const bool has_src = !a.reverse && src.find(a.t0);
     const bool top = !INNER && i0 <= 0 && i0 + R > 0;  // the wave holds row 0
     const bool surf_here = top && a.reverse && a.surf;
 
@@ -127,17 +122,7 @@ __device__ __forceinline__ void sponge2d_tile(const Sponge2dArgs &a, int tx, int
     auto sources = [&](int t, float (&sv)[R]) {
 #pragma unroll
         for (int r = 0; r < R; ++r) sv[r] = 0.f;
-        if (has_src && t < a.src_nt)
-            for (int k = 0; k < a.nsrc; ++k) {
-                const int cell = ld_uniform(a.src_cell + k);
-                const int ci = cell / a.nx, cj = cell - ci * a.nx;
-                const float amp = ld_uniform(a.src_amp + (size_t)t * a.nsrc + k);
-                if (cj == j) {
-#pragma unroll
-                    for (int r = 0; r < R; ++r)
-                        if (ci == i0 + r) sv[r] += amp;
-                }
-            }
+        if (has_src) src.add(t, j, sv);
         if (surf_here && t < a.surf_nt) {
             const float x = jin ? a.surf[(size_t)t * a.nx + j] : 0.f;
 #pragma unroll
@@ -146,9 +131,9 @@ __device__ __forceinline__ void sponge2d_tile(const Sponge2dArgs &a, int tx, int
         }
     };
     const bool driven = has_src || surf_here;  // wave-uniform
-    auto update = [&](float (&p)[R], float (&q)[R], float up, float below, int t, auto src) {
+    auto update = [&](float (&p)[R], float (&q)[R], float up, float below, int t, auto drive) {
         float sv[R];
-        if constexpr (src) sources(t, sv);
+        if constexpr (drive) sources(t, sv);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const float pc = p[r], dn = r + 1 < R ? p[r + 1] : below;
@@ -157,7 +142,7 @@ __device__ __forceinline__ void sponge2d_tile(const Sponge2dArgs &a, int tx, int
             // rounding then scales with the increments instead of with 2p.
             float lap = fmaf(ax[r], (lane_right(pc) - pc) + (lane_left(pc) - pc),
                              az[r] * ((dn - pc) + (up - pc)));
-            if constexpr (src) {
+            if constexpr (drive) {
                 const float vd = iin(r) && jin ? a.vdt[(size_t)(i0 + r + kHZ) * a.pitch + j + kHX]
                                                : 0.f;
                 lap = fmaf(-sv[r], vd * vd, lap);
@@ -237,7 +222,7 @@ __device__ __forceinline__ void sponge2d_tile(const Sponge2dArgs &a, int tx, int
 // full chip: 100 x 150 1.14 against 1.50 ms, 515 x 1203 3.43 against 2.85.
 // Blocks are 1-D over the tiles, XCD-banded: block b runs on XCD b % 8 and
 // takes the next tile of that XCD's contiguous band.
-template <int R>
+template <int R, bool MANY>
 __global__ void __launch_bounds__(64 * kSpZ / R) sponge2d_steps(Sponge2dArgs a, int ntx) {
     __shared__ float edge[2][kSpZ / R + 2][2][64];
     const int nb = (int)gridDim.x, b = (int)blockIdx.x;
@@ -246,9 +231,9 @@ __global__ void __launch_bounds__(64 * kSpZ / R) sponge2d_steps(Sponge2dArgs a, 
     const int ty = t / ntx, tx = t - ty * ntx;
     const int z0 = ty * kSpCZ - kSpK, x0 = tx * kSpCX - kSpK;  // first row and column held
     if (z0 > 0 && z0 + kSpZ <= a.nz - a.nB && x0 >= a.nB && x0 + 64 <= a.nx - a.nB)
-        sponge2d_tile<R, true>(a, tx, ty, edge);
+        sponge2d_tile<R, true, MANY>(a, tx, ty, edge);
     else
-        sponge2d_tile<R, false>(a, tx, ty, edge);
+        sponge2d_tile<R, false, MANY>(a, tx, ty, edge);
 }
 
 // One time step: for runs cut into pieces of a step or two, where the tiles of
@@ -307,17 +292,10 @@ __global__ void __launch_bounds__(256) sponge2d_step(Sponge2dArgs a, int ntx) {
     float s[RZ];
 #pragma unroll
     for (int r = 0; r < RZ; ++r) s[r] = 0.f;
-    if (!a.reverse && t < a.src_nt)
-        for (int k = 0; k < a.nsrc; ++k) {
-            const int cell = ld_uniform(a.src_cell + k);
-            const int ci = cell / a.nx, cj = cell - ci * a.nx;
-            if (ci >= i0 && ci < i0 + RZ && cj == j) {
-                const float amp = ld_uniform(a.src_amp + (size_t)t * a.nsrc + k);
-#pragma unroll
-                for (int r = 0; r < RZ; ++r)
-                    if (ci == i0 + r) s[r] += amp;
-            }
-        }
+    if (!a.reverse && a.nsrc > 0) {
+        WaveSources<RZ, true> src{a.src_cell, a.src_amp, a.nsrc, a.src_nt, a.nx, i0, tx * 64};
+        if (src.find(t)) src.add(t, j, s);
+    }
     if (a.reverse && a.surf && t < a.surf_nt && i0 == 0 && jin) s[0] += a.surf[(size_t)t * a.nx + j];
     float *snap = a.snap && t % a.snap_stride == 0
                       ? a.snap + (size_t)(t / a.snap_stride - a.snap_slot0) * a.nz * a.nx
@@ -679,10 +657,11 @@ class Prop2D final : public Prop {
         // 4 rows per wave while the tiles (8 waves each) leave the chip's 1024
         // SIMDs idle or nearly so, 8 rows from two blocks per CU
         const dim3 grid((unsigned)(ntx * ntz));
-        if (ntx * ntz < 512)
-            hipLaunchKernelGGL(sponge2d_steps<4>, grid, dim3(64 * kSpZ / 4), 0, stream, a, ntx);
-        else
-            hipLaunchKernelGGL(sponge2d_steps<8>, grid, dim3(64 * kSpZ / 8), 0, stream, a, ntx);
+        const dim3 block(64 * kSpZ / (ntx * ntz < 512 ? 4 : 8));
+        auto kernel = a.nsrc > kFewSources
+                          ? (ntx * ntz < 512 ? sponge2d_steps<4, true> : sponge2d_steps<8, true>)
+                          : (ntx * ntz < 512 ? sponge2d_steps<4, false> : sponge2d_steps<8, false>);
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, a, ntx);
         SSSI_HIP(hipGetLastError());
         cur ^= 1;
         return 1;

@@ -70,3 +70,26 @@ def test_sponge_pieces(nz, nx, n, single, several):
     """Pieces of one step, and of two on a full chip, take the one-step kernel."""
     out = hipmock.run(_SPONGE.format(nz=nz, nx=nx, n=n)).split()
     assert [int(x) for x in out] == [single, several]
+
+
+_SOURCES = """
+v = np.full((100, 150), 2000.0, order="F")
+P = sssi_amd.Propagator(v, {N}, 5, 10.0, 10.0, 1e-3, abc="{abc}")
+k = np.arange({n})
+P.set_points(k // 150, k % 150, np.zeros((16, {n})))
+M.hipmock_clear()
+P.run_steps(0, 16)
+print(count("steps") - count("ELb1EE"), count("ELb1EE"))
+"""
+
+
+@pytest.mark.parametrize("abc, N, n, few, many", [
+    ("sponge", 1, 4, 2, 0), ("sponge", 1, 5, 0, 2), ("sponge", 1, 2000, 0, 2),
+    ("cpml", 1, 4, 2, 0), ("cpml", 1, 5, 0, 2), ("cpml", 2, 8, 4, 0), ("cpml", 2, 9, 0, 4),
+    ("cpml", 2, 64, 0, 4), ("cpml", 2, 65, 0, 0),
+])
+def test_sources_per_launch(abc, N, n, few, many):
+    """Launches of several steps that loop over all sources, and that test 64 at
+    a time; CPML with more than 64 sources takes its one-step kernel."""
+    out = hipmock.run(_SOURCES.format(abc=abc, N=N, n=n)).split()
+    assert [int(x) for x in out] == [few, many]
