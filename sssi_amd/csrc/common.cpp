@@ -2,6 +2,7 @@
 #include "common.h"
 
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstring>
 #include <map>
@@ -218,27 +219,37 @@ struct PinnedChunk {
 struct Relay {
     std::mutex mu;
     std::condition_variable go, through;
-    bool stop = false;
-    size_t ready = 0, team = 0;  // chunks that have come; workers there are
+    std::atomic<bool> stop{false};
+    std::atomic<size_t> ready{0};  // chunks that have come
+    long team = -1;                // workers that take part (-1: not decided)
+    // A chunk that is on its way comes within 0.2 ms: a worker looks for it that
+    // long before it goes to sleep, as waking 15 takes 50 us.
+    void look(size_t c) const {
+        const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+        while (ready.load() <= c && !stop.load() && std::chrono::steady_clock::now() < until)
+            std::this_thread::yield();
+    }
     std::vector<size_t> done;    // workers that are through with a chunk
 };
 
 // Workers of all calls of the process at a time: they widen and page in
 // results, which is bound by the host's memory and its page tables.  Four and
 // eight threads bringing 24 MB each to the host: 2.5 and 4.8 ms with 15 workers
-// a call, 1.9 and 2.4 with 15 in all.
-constexpr long kWorkers = 15;
-std::atomic<long> g_workers{0};
+// a call, 1.9 and 2.4 with 15 in all.  They are started while the stream still
+// computes (starting 15 takes 0.3 ms) and asleep until it is done, and only then
+// is it decided how many take part.
+constexpr long kWorkers = 15, kAsleep = 60;
+std::atomic<long> g_workers{0}, g_asleep{0};
 
 // The workers; left early (an exception), they are told to stop and joined.
 struct Crew {
     Relay &r;
     std::vector<std::thread> th;
-    long taken = 0;  // of kWorkers
+    long held = 0, taken = 0;  // of kAsleep, of kWorkers
     template <class F>
     void start(size_t want, F &f) {
-        taken = (long)want;
-        const long n = std::min<long>(taken, kWorkers - g_workers.fetch_add(taken));
+        held = (long)want;
+        const long n = std::min<long>(held, kAsleep - g_asleep.fetch_add(held));
         if (n < 2) return;
         try {
             th.reserve((size_t)n);
@@ -246,8 +257,18 @@ struct Crew {
         } catch (const std::system_error &) {  // no more threads: those there do it
         } catch (const std::bad_alloc &) {
         }
-        std::lock_guard<std::mutex> lk(r.mu);
-        r.team = th.size();
+    }
+    // How many take part (0: the caller does it); the others leave.
+    long decide() {
+        taken = (long)th.size();
+        const long n = std::min<long>(taken, kWorkers - g_workers.fetch_add(taken));
+        const long team = n < 2 ? 0 : n;
+        {
+            std::lock_guard<std::mutex> lk(r.mu);
+            r.team = team;
+        }
+        r.go.notify_all();
+        return team;
     }
     void join() {
         for (auto &t : th)
@@ -261,6 +282,7 @@ struct Crew {
         r.go.notify_all();
         join();
         g_workers -= taken;
+        g_asleep -= held;
     }
 };
 }  // namespace
@@ -277,8 +299,6 @@ void stream_to_host(const void *dev, size_t n, size_t elem, hipStream_t s, const
                                 std::min(per, n - c * per) * elem, hipMemcpyDeviceToHost, s));
         SSSI_HIP(hipStreamSynchronize(s));
     };
-    // what the stream still computes, before any worker waits for it
-    SSSI_HIP(hipStreamSynchronize(s));
     // a worker per MB, up to 15; none for a small result
     const size_t want = std::min<size_t>({15, n * elem >> 20,
                                           std::max(1u, std::thread::hardware_concurrency())});
@@ -286,10 +306,16 @@ void stream_to_host(const void *dev, size_t n, size_t elem, hipStream_t s, const
     r.done.assign(nchunk, 0);
     auto work = [&](size_t k) {
         std::unique_lock<std::mutex> lk(r.mu);
+        r.go.wait(lk, [&] { return r.stop || r.team >= 0; });
+        const long team = r.team;
+        if (r.stop || (long)k >= team) return;
+        const size_t T = (size_t)team;
         for (size_t c = 0; c < nchunk; ++c) {
-            r.go.wait(lk, [&] { return r.stop || (r.team > 0 && r.ready > c); });
+            lk.unlock();
+            r.look(c);
+            lk.lock();
+            r.go.wait(lk, [&] { return r.stop || r.ready > c; });
             if (r.stop) return;
-            const size_t T = r.team;
             lk.unlock();
             const size_t m = std::min(per, n - c * per), a = m * k / T, b = m * (k + 1) / T;
             if (b > a) use((const char *)buf[c & 1].p + a * elem, c * per + a, b - a);
@@ -298,8 +324,12 @@ void stream_to_host(const void *dev, size_t n, size_t elem, hipStream_t s, const
         }
     };
     Crew crew{r};  // (last: joined before anything the workers use is gone)
-    if (want > 1) crew.start(want, work);
-    const size_t T = crew.th.size();
+    size_t T = 0;  // that take part
+    if (want > 1) {
+        crew.start(want, work);
+        SSSI_HIP(hipStreamSynchronize(s));  // what the stream still computes
+        T = (size_t)crew.decide();
+    }
     for (size_t c = 0; c < nchunk; ++c) {
         if (T > 0 && c >= 2) {  // the buffer's last chunk has been used
             std::unique_lock<std::mutex> lk(r.mu);

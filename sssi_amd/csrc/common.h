@@ -160,8 +160,8 @@ struct HostBuf {
 // while worker threads hand the chunk before to use(src, first, count), which
 // puts elements first .. first+count-1 (at src) where they belong.  use is
 // called from several threads on disjoint ranges and must not throw.  Returns
-// when everything has been used.  The threads sleep while a chunk is on its
-// way, and none is there yet while the stream's earlier work runs.  A fresh result array costs a page fault per
+// when everything has been used.  The threads sleep while the stream's
+// earlier work runs, and look for at most 0.2 ms for a chunk on its way.  A fresh result array costs a page fault per
 // 4 KB and a pageable copy takes them one by one on the runtime's own staging:
 // 92 MB of traveltimes took 11 ms as one hipMemcpy and take 4 this way.
 using HostUse = std::function<void(const void *src, size_t first, size_t count)>;
