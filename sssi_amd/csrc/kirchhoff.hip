@@ -101,7 +101,7 @@ __device__ __forceinline__ double wave_shl1(double v) {
 // change in the previous launch would compute its present values again; they
 // stand in both levels already.  (A launch that changed nothing at H passes
 // changes nothing at fewer: every pass takes a minimum with the old value.)
-// The first launch runs every tile (list null), with both levels initialised.
+// The first launch runs every tile (list null), which also fills the other level.
 // A tile that changed puts itself and its neighbours in the next launch's
 // list, each once (`mark` holds the stamp of the launch a tile was last put
 // in the list for).  The order of the list does not affect any value.
@@ -531,9 +531,6 @@ class Eikonal2D {
             mark.alloc((size_t)nblk);
             fill_int(counts.p, counts.n, 0, stream);
             fill_int(mark.p, mark.n, 0, stream);
-            if (nlaunch > 0)
-                hipLaunchKernelGGL(eik_init, dim3(grid_blocks(total)), dim3(256), 0, stream,
-                                   t[1].p, nn, nsrc, src.p);
             const dim3 grid((unsigned)std::min<int64_t>(nblk, kEikBlocks));
             for (int p = 0; p < 4 * iMax; p += lay.h) {
                 const int np = std::min(lay.h, 4 * iMax - p);

@@ -93,3 +93,14 @@ def test_sources_per_launch(abc, N, n, few, many):
     a time; CPML with more than 64 sources takes its one-step kernel."""
     out = hipmock.run(_SOURCES.format(abc=abc, N=N, n=n)).split()
     assert [int(x) for x in out] == [few, many]
+
+
+@pytest.mark.parametrize("layout", ["8x24", "4x32", "plain"])
+def test_eikonal_fills_one_level(layout):
+    """The first launch writes every cell of the other level."""
+    out = hipmock.run("""
+V = np.full((90, 70), 2000.0, order="F")
+sssi_amd.eikonal2d_batch(V, 10.0, [1, 1], [3, 60], 12)
+print(count("eik_init"))
+""", SSSI_EIK=layout)
+    assert int(out) == 1
