@@ -503,8 +503,9 @@ class Eikonal2D {
                            nsrc, iMax > 0 ? src.p : nullptr);
         SSSI_HIP(hipGetLastError());
         cur = 0;
-        // work lists (EikList): two lists, the launches' counts, the marks
-        DevBuf<int> lists, counts, mark;
+        // work lists (EikList): the launches' counts, the marks, two lists; in one
+        // buffer, as every free waits for all of the device's callers
+        DevBuf<int> work;
         const double dxi = (double)(int)dx;  // eikonal2d_mex.cpp:35 reads dx as an int
         hipEvent_t ev[2];
         SSSI_HIP(hipEventCreate(&ev[0]));
@@ -526,18 +527,15 @@ class Eikonal2D {
             if (nblk > INT32_MAX) fail(SSSI_EINVAL, "too many traveltime tables for one launch");
             launches = 0;
             const int64_t nlaunch = (4 * (int64_t)iMax + lay.h - 1) / lay.h;
-            lists.alloc((size_t)(2 * nblk));
-            counts.alloc((size_t)nlaunch + 1);
-            mark.alloc((size_t)nblk);
-            fill_int(counts.p, counts.n, 0, stream);
-            fill_int(mark.p, mark.n, 0, stream);
+            work.alloc((size_t)nlaunch + 1 + (size_t)(3 * nblk));
+            int *const counts = work.p, *const mark = counts + nlaunch + 1, *const lists = mark + nblk;
+            fill_int(counts, (size_t)nlaunch + 1 + (size_t)nblk, 0, stream);
             const dim3 grid((unsigned)std::min<int64_t>(nblk, kEikBlocks));
             for (int p = 0; p < 4 * iMax; p += lay.h) {
                 const int np = std::min(lay.h, 4 * iMax - p);
                 const int n = (int)launches;
-                const EikList w{n ? lists.p + (size_t)(n & 1) * nblk : nullptr, counts.p + n,
-                                lists.p + (size_t)((n & 1) ^ 1) * nblk, counts.p + n + 1, mark.p,
-                                n + 1};
+                const EikList w{n ? lists + (size_t)(n & 1) * nblk : nullptr, counts + n,
+                                lists + (size_t)((n & 1) ^ 1) * nblk, counts + n + 1, mark, n + 1};
                 lay.launch(n ? grid : dim3((unsigned)nblk), stream, slow.p, t[cur].p,
                            t[cur ^ 1].p, (int)nz, (int)nx, ntz, ntx, nsrc, src.p, dxi, np, w);
                 SSSI_HIP(hipGetLastError());
