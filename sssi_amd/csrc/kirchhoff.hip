@@ -371,8 +371,10 @@ __global__ void __launch_bounds__(64) kirch_group(const int *__restrict__ kidx, 
             const int64_t c = (int64_t)xr[min(r0 + v, nrec - 1)] * nt;
 #pragma unroll
             for (int u = 0; u < S; ++u) {
-                // 0-based sample (1-based indices ks, kn); both below 2^31
-                const uint32_t it = ks[u] + kn[v] - 1u;
+                // 0-based sample (1-based signed indices ks, kn, added modulo 2^32):
+                // below nt < 2^29 only where the sum is, or where both are
+                // negative and it wraps round, which the sign bit keeps out
+                const uint32_t it = (ks[u] + kn[v] - 1u) | (ks[u] & kn[v] & 0x80000000u);
                 const bool in = it < nt;
                 oob |= live && !in;
                 ok[v][u] = live && in;
