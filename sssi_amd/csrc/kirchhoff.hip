@@ -626,10 +626,16 @@ static float kirchhoff_run(const int *kidx_dev, int64_t nz, int64_t nx, int64_t 
     for (int r = 0; r < nrec; ++r) xr0[r] = xrec[r] - 1;
     const int64_t nn = nz * nx;
     // shot groups in parallel, then the stack in shot order, when their images
-    // fit a scratch buffer and a trace a 32-bit byte offset
+    // fit a scratch buffer, a trace a 32-bit byte offset and the patches a grid
+    // (fewer than 2^32 threads; a patch of a model of one row is mostly empty).
+    // SSSI_KIRCH=stack: the form without groups everywhere.
+    const int64_t ntz = (nz + kKirchZ - 1) / kKirchZ;
+    const int64_t ntx = (nx + 64 / kKirchZ - 1) / (64 / kKirchZ);
     const int ngroups = (nshot + kShotGroup - 1) / kShotGroup;
+    const char *form = std::getenv("SSSI_KIRCH");
     const bool grouped = ngroups <= 65535 && (double)nn * nshot * 8 <= 4e9 &&
-                         nt < ((int64_t)1 << 29);
+                         nt < ((int64_t)1 << 29) && ntz * ntx < ((int64_t)1 << 26) &&
+                         !(form && !std::strcmp(form, "stack"));
     KirchWork local;
     KirchWork &w = work ? *work : local;
     const bool pinned = work != nullptr;  // a one-shot call copies straight to the caller
@@ -644,14 +650,12 @@ static float kirchhoff_run(const int *kidx_dev, int64_t nz, int64_t nx, int64_t 
     hipEvent_t *ev = w.ev;
     SSSI_HIP(hipEventRecord(ev[0], s));
     if (grouped) {
-        const int ntz = (int)((nz + kKirchZ - 1) / kKirchZ);
-        const int64_t ntx = (nx + 64 / kKirchZ - 1) / (64 / kKirchZ);
         const int per = (nshot + ngroups - 1) / ngroups;  // equal groups
         const dim3 grid((unsigned)(ntz * ntx), (unsigned)((nshot + per - 1) / per));
 #define SSSI_KIRCH_CASE(S_, U_)                                                              \
     case S_:                                                                                 \
         hipLaunchKernelGGL((kirch_group<S_, U_>), grid, dim3(64), 0, s, kidx_dev, (int)nz,   \
-                           (int)nx, ntz, dts, nshot, dtr, dxr, nrec, dshots, (uint32_t)nt,   \
+                           (int)nx, (int)ntz, dts, nshot, dtr, dxr, nrec, dshots, (uint32_t)nt,   \
                            w.img.p, w.bad.p);                                                \
         break;
         switch (per) {
