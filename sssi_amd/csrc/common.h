@@ -39,13 +39,17 @@ const char *last_error_text();
     throw Error(code, buf);
 }
 
+// (The runtime keeps a thread's last error until it is asked for; a failure that
+// is reported here must not be found again behind the next call's launch.)
 #define SSSI_HIP(call)                                                                  \
     do {                                                                                \
         hipError_t e_ = (call);                                                         \
-        if (e_ != hipSuccess)                                                           \
+        if (e_ != hipSuccess) {                                                         \
+            (void)hipGetLastError();                                                    \
             ::sssi::fail(e_ == hipErrorOutOfMemory ? SSSI_ENOMEM : SSSI_EDEVICE,        \
                          "%s failed: %s (%s:%d)", #call, hipGetErrorString(e_),         \
                          __FILE__, __LINE__);                                           \
+        }                                                                               \
     } while (0)
 
 // Stream of the stream-ordered allocator for the calling thread's device

@@ -35,11 +35,14 @@ std::atomic<size_t> mem_free{(size_t)1 << 38};
 dim3 cfg_grid, cfg_block;
 int dummy;
 
+// hipGetLastError's: the thread's last failure, until it is asked for (a call
+// that succeeds does not clear it)
+thread_local hipError_t last = hipSuccess;
 thread_local long new_in = -1;  // this thread's operator new calls until one throws
 
 hipError_t take(void **p, size_t n) {
     ++n_malloc;
-    if (fail_in >= 0 && fail_in-- == 0) return hipErrorOutOfMemory;
+    if (fail_in >= 0 && fail_in-- == 0) return last = hipErrorOutOfMemory;
     *p = std::calloc(n ? n : 1, 1);
     std::lock_guard<std::mutex> lk(mu);
     sizes[*p] = n;
@@ -142,6 +145,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, h
     launches.push_back(std::move(l));
     // (the runtime's limit: fewer than 2^32 threads in a dimension)
     const bool fits = (unsigned long long)g.x * b.x < (1ull << 32) && g.x && g.y && g.z;
+    if (!fits) last = hipErrorInvalidConfiguration;
     return fits ? hipSuccess : hipErrorInvalidConfiguration;
 }
 hipError_t hipMalloc(void **p, size_t n) { return take(p, n); }
@@ -195,7 +199,11 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int) {
     p->multiProcessorCount = 256;
     return hipSuccess;
 }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    const hipError_t e = last;
+    last = hipSuccess;
+    return e;
+}
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
 hipError_t hipGetSymbolAddress(void **p, const void *) { *p = std::calloc(64 << 20, 1); return hipSuccess; }
 hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t *p, int) { *p = nullptr; return hipSuccess; }
