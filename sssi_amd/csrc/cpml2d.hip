@@ -738,9 +738,13 @@ __global__ void step_base_add(int *base, int k) {
 // after n <= K steps the inner CZ x CX cells are exact and are what the tile
 // writes, into buffers other than those its neighbours still read.  Cells
 // outside the model stay 0, which is the boundary.
-// Bound by vector issue: the step kernel takes ~7 us per step on these grids
-// whatever their size, this one ~5 us per launch and then ~1.2 us (N = 1) to
-// ~3 us (N = 4) per step and round of workgroups.  120 x 240 cells, 600 steps,
+// Bound by latency within a workgroup: a wavefront of a 120 x 240 launch spends
+// 40 to 43 % of its life waiting (LDS, barriers, the first loads), 18 to 26 %
+// waiting to issue and 18 to 23 % issuing vector instructions, with two (N = 3:
+// three) wavefronts to a SIMD; 130 to 162 scalars spilled to vector lanes are
+// part of both.  The step kernel takes ~7 us per step on these grids whatever
+// their size, this one ~5 us per launch and then ~1.2 us (N = 1) to ~3 us (N =
+// 4) per step and round of workgroups.  120 x 240 cells, 600 steps,
 // whole call, one step per launch -> this kernel: N=1 4.08 -> 1.37 ms, N=2 4.08
 // -> 2.00, N=3 4.20 -> 3.29, N=4 4.31 -> 3.54; 300 x 500 cells: N=1 4.23 ->
 // 1.62, N=2 4.34 -> 2.77, N=3 4.37 -> 3.74.  K and W are the best of a sweep
@@ -1429,7 +1433,11 @@ void launch_cpml2d_batch(int N, int rz, int ng, const Job2D *jobs, const int2 *o
 // tiles 5.83 vs 6.39; N=2 645 tiles (340 x 600) 4.37 vs 3.50, 850 tiles 4.55 vs
 // 4.64; N=3 255 tiles (300 x 500) 4.30 vs 3.75, 306 tiles 4.39 vs 5.09; N=4 240
 // tiles (118 x 270) 4.33 vs 3.48, 264 tiles 4.85 vs 6.00 (here and at N=3 a CU
-// holds one workgroup, and the 257th starts a second round).
+// holds one workgroup, and the 257th starts a second round).  The line is drawn
+// for one call at a time: handles that share the chip also share the rim's work,
+// which at N=4 costs more than the launches it saves (118 x 240, 400 steps each,
+// one step per launch vs several, ms: 1 handle 2.75 vs 2.26, 4 handles 5.6 vs
+// 6.2, 8 handles 8.6 vs 10.7; at N=2, 8 handles 8.1 vs 3.8).
 template <int N>
 static int steps_rule(const Cpml2dGrid &g) {
     using T = Steps2D<N>;

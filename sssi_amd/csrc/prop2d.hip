@@ -426,8 +426,9 @@ class Prop2D final : public Prop {
         SSSI_HIP(hipMemcpy(order.p, ord.data(), order.bytes(), hipMemcpyHostToDevice));
     }
 
-    // Autotuner: time every instantiated layout (tile height, march groups) on
-    // this grid -- kTuneSteps launches after a short warm-up, HIP events on the
+    // Autotuner of the step kernel (small grids run most of their steps several to
+    // a launch, where only the stencil forms of its tile height are kept): time
+    // every instantiated layout (tile height, march groups) on this grid -- kTuneSteps launches after a short warm-up, HIP events on the
     // handle's stream -- keep the fastest, and cache it for the shape.
     void tune_layout() {
         const TuneKey key{2, nz, nx, 1, N, nB};

@@ -902,6 +902,8 @@ class Prop3D final : public Prop {
             zc = b;
             return;
         }
+        // (The candidates are for large grids: up to 640 blocks of 32 planes the
+        // default chunk of 8 or 24 planes is faster than any of them.)
         // z chunks: at 420 x 440 x 440, 8-row tiles, us per step at 48, 64, 80, 96,
         // 112 planes: 457.6, 461.7, 454.2, 472.8, 472.5 (one box)
         static const int cty[] = {4, 8, 16};
@@ -1065,7 +1067,11 @@ class Prop3D final : public Prop {
     // 78 / 85 / 96; 300 (160^3) 56 / 56 / 62 / 79; 432 (180 x 190 x 190) 71 / 74 / 66 /
     // 81; 600 (170 x 250 x 200) 84 / 76 / 80 / 84; 700 (200^3, order 2) 86 / 87 / 89 /
     // 84; 784 (220 x 250 x 220) 113 / 104 / 103 / 105; 5390 (420 x 440 x 440)
-    // 591 / 529 / 504 / 490.
+    // 591 / 529 / 504 / 490.  The rule's chunk against 32 planes at order 8, whose
+    // blocks start up on 30 planes outside their chunk: 64^3 35 / 102, 100 x 200 x
+    // 120 98 / 107, 160^3 125 / 148, 180 x 190 x 190 146 / 175.  Handles that run at
+    // once pay for the start-ups instead: 8 of 160^3, order 3, 31.5 against 28.0 ms
+    // for 100 steps (one alone 4.7 against 6.8), 8 of 128^3, order 4, 17.4 / 23.4.
     int default_chunk() const {
         const int64_t blocks =
             ((nx + kTX - 1) / kTX) * ((ny + ty - 1) / ty) * ((nz + 31) / 32);
