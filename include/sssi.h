@@ -55,7 +55,10 @@ int sssi_set_device(int device);
  * appended to the file named by SSSI_TUNE_CACHE, if set).  Off by default
  * (SSSI_AUTOTUNE=1 turns it on); results of different layouts agree with the
  * oracle to the same tolerance, and may differ from each other in the last
- * bits near damping-strip edges. */
+ * bits near damping-strip edges.
+ * The 3-D candidates are z chunks of 32 to 128 planes, for large grids; up to
+ * 640 blocks of 64 x 8 x 32 cells the untuned default (8 or 24 planes) is faster
+ * than any of them. */
 int sssi_set_autotune(int on);
 
 /* ---------------------------------------------------------------------
