@@ -107,12 +107,16 @@ for _ in range(8):
     P.set_points([0], [1], np.zeros(1000))
     P.run(1000)
     Ps.append(P)
-M.hipmock_sync_us(20000)  # every call holds its chunks while the others start
+M.hipmock_sync_us(100000)  # every call holds its chunks while the others start
 def once():
-    th = [threading.Thread(target=P.data, args=(1000,)) for P in Ps]
+    bar = threading.Barrier(8)
+    def call(P):
+        bar.wait()
+        P.data(1000)
+    th = [threading.Thread(target=call, args=(P,)) for P in Ps]
     for t in th: t.start()
     for t in th: t.join()
-once()
+once(); once()
 n = M.hipmock_host_mallocs()
 for _ in range(3): once()
 print(M.hipmock_host_mallocs() - n)
@@ -120,6 +124,6 @@ print(M.hipmock_host_mallocs() - n)
 
 
 def test_concurrent_calls_find_their_chunks():
-    """Eight callers at a time: after the first round no pinned memory is
+    """Eight callers at a time: after the first rounds no pinned memory is
     allocated."""
     assert int(hipmock.run(_POOL)) == 0
